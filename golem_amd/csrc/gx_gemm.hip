@@ -17,9 +17,8 @@
 // so it comes from the matrix core too: v_mfma_f32_32x32x8_f16 with the two
 // vectors in k = 0 and zeros elsewhere gives every product exactly (an
 // 11-bit by 11-bit product fits fp32; the int8 kernel puts them in k = 0 and
-// k = 4 and takes 2 d_w d_a against half the integer).  The vector ALU is
-// left with one conversion (a subtraction) and one fma per element per
-// block.
+// k = 4 and takes 2 d_w d_a).  The vector ALU is left with one fma per
+// element per block.
 //
 // Two kernels: the int8 one below (loads straight into LDS, every Q4_0
 // product of more than a few tokens, dense or grouped by expert) and an fp16
@@ -316,73 +315,58 @@ __global__ __launch_bounds__(64 * NWT) void q4_0_gemm_f16_kernel(
 
 // ---- the int8 product, loads straight into LDS -------------------------
 //
-// The kernel for the Q4_0 x Q8_0 product of a batch.  Every stage's operands come in by direct
-// global-to-LDS loads (global_load_lds_dwordx4 / _dword): no registers stage
-// them, and the stages live in an LDS ring of kRing slots (four for the
-// 64-token form, three for the 32-token one), all but one in flight while one
-// is multiplied.  A workgroup owns 128 rows (two R64 tiles) x 64 tokens; each
-// of its eight wavefronts one 32x32 MFMA tile (rows 32*(w&3), tokens
-// 32*(w>>2)), at four wavefronts per SIMD (two workgroups per CU).  Per stage
-// (4 blocks) each wavefront issues exactly kLoads loads, so `s_waitcnt
-// vmcnt((kRing - 2) kLoads)` before the stage's barrier means "this stage has
-// landed" for every wavefront; the barrier is the bare s_barrier (the fence of
-// __syncthreads would wait for every load in flight).  Slot layout (bytes):
-//   [0, 8192)       nibbles  [block 4][row 128][16]
-//   [8192, 16384)   int8     [block 4][half 2][token 64][16]
-//   [16384, 17408)  act. scales (fp32) [block 4][token 64]
-//   [17408, 18432)  weight scales (fp16) [row 128][block 4]
-constexpr int kDmaTok = 64;
-// LDS slots of the ring (stages in flight + 1).  The 64-token form takes
-// four (two workgroups a CU still fit: 2 x 72 KiB): config 2 at M = 2048
-// 180 -> 177 us; the 32-token form keeps three, which keep three
-// workgroups a CU (four slots: M = 512 50 -> 55 us, config 4's prefill
-// 181 -> 189 us).
-#ifndef GX_DMA_RING64
-#define GX_DMA_RING64 4
-#endif
-#ifndef GX_DMA_RING32
-#define GX_DMA_RING32 3
-#endif
-// The integer products run on a biased chain.  The weights enter the MFMA as
-// 16 * (n - 8) (the nibble in a byte's high half, its top bit flipped), and
-// each block's MFMA adds its 16 * isum to the previous block's output; a
-// stretch's chain starts from the bits of 1.5 * 2^18.  Read as fp32, every
-// output is then 1.5 * 2^18 plus half the stretch's running isum, exactly:
-// the ulp in [2^18, 2^19) is 1/32, and the running sum of a stretch is at
-// most 8 blocks * 32 * 8 * 128 = 2^18 in magnitude, 2^22 ulps either side of
-// the middle of the binade, whose ends (bits 0x48800000 and 0x49000000) are
-// exactly 2^18 and 2^19.  The difference of two consecutive outputs is half
-// the block's isum as an fp32 -- one full-rate subtraction instead of a
-// conversion -- and the scale outer product is 2 d_w d_a (k04_operand), so
-// fma(isum / 2, 2 d_w d_a, acc) is golem's fma(isum, d_w d_a, acc) bit for
-// bit: the two products are the same real number, rounded once.
-constexpr int kChainBias = 0x48C00000;  // 393216.0f
-
-// One block's operands from LDS (nibbles, activations, weight scale,
-// activation scale), issued without a wait.  Written out so that the
-// compiler sees no LDS load: it would otherwise make each one wait for every
-// load-to-LDS in flight, the next stages' included.  The caller waits
-// (lgkmcnt) before it uses the four registers.
+// The kernel for the Q4_0 x Q8_0 product of a batch.  Every stage's operands
+// come in by direct global-to-LDS loads (global_load_lds_dwordx4 / _dword):
+// no registers stage them, and the stages live in an LDS ring of kRing slots,
+// all but one in flight while one is multiplied.  Per stage (4 blocks) each
+// wavefront issues exactly kLoads loads, so `s_waitcnt vmcnt((kRing - 2)
+// kLoads)` before the stage's barrier means "this stage has landed" for every
+// wavefront; the barrier is the bare s_barrier (the fence of __syncthreads
+// would wait for every load in flight).  A stage's loads go out one or two a
+// tile, and a block's operands are read from LDS a block ahead, across
+// stages.
 //
-// Lane (row or token l % 32, half g = l / 32) reads 8 bytes of its row's
-// nibble chunk, bytes 8g .. 8g + 7, and takes both nibbles of each: its MFMA
-// slots are k = 16 + 8g .. 16 + 8g + 7 (the high nibbles) then k = 8g ..
-// 8g + 7 (the low ones), and its activation operand holds the same k in the
-// same order: bytes 8g .. 8g + 7 of the block's second half (OA1), then of
-// its first half (OA0).  The integer sum does not depend on the order of k;
-// a lane widening a whole half-chunk's one nibble needed two instructions a
-// dword for the low half, and this takes six for the lane's sixteen.
-template <int OW, int OA1, int OA0, int OD, int OS>
-__device__ __forceinline__ void lds_read_block(uint32_t aw, uint32_t aa, uint32_t ad, uint32_t as, uint2 &rw,
-                                               uint2 &ra1, uint2 &ra0, uint32_t &rdw, float &rda) {
-    asm volatile(
-        "ds_read_b64 %0, %5 offset:%9\n\t"
-        "ds_read_b64 %1, %6 offset:%10\n\t"
-        "ds_read_b64 %2, %6 offset:%11\n\t"
-        "ds_read_u16 %3, %7 offset:%12\n\t"
-        "ds_read_b32 %4, %8 offset:%13"
-        : "=&v"(rw), "=&v"(ra1), "=&v"(ra0), "=&v"(rdw), "=&v"(rda)
-        : "v"(aw), "v"(aa), "v"(ad), "v"(as), "i"(OW), "i"(OA1), "i"(OA0), "i"(OD), "i"(OS));
+// What bounds it: a tile and block take three MFMAs (96 cycles of the matrix
+// core) and about 23 vector instructions, which mostly add up; under that
+// load the clock is 2.1 GHz.  Taken out of a copy, the loads changed 126 us
+// to 122 and the stores to 114 (9728 x 2560 at 2048 tokens).  With a token a
+// lane in the activation's loads, the subtraction on the vector ALU and one
+// 32x32 tile a wavefront throughout the same product took 175 us (0.117 of
+// the int8 rate; now 0.162), 49 at 500 tokens (now 38), 2560 x 9728 at 500 64
+// (now 51), a mixture layer of 128 experts at 256 positions 175 (159).
+//
+// The integer products are taken as floats without a conversion.  The weights
+// enter the MFMA as 16 * (n - 8) (the nibble in a byte's high half, its top
+// bit flipped) and its addend is the bits of 0.1875, the middle of the binade
+// [1/8, 1/4): a block's 16 * isum is at most 16 * 32 * 8 * 128 = 2^19 in
+// magnitude, 2^3 less than the 2^22 ulps to either end, so the output read as
+// fp32 is 0.1875 + 16 * isum * 2^-26 exactly, and no block waits for the one
+// before it.  A second MFMA (1 * -0.1875 added to that output) leaves
+// isum * 2^-22 exactly: a sixteen-instruction subtraction taken off the
+// vector ALU, whose instructions, not the matrix core's, bound the product
+// (the two units' times add up on a SIMD; 57 -> 52 ns a tile and block).  The
+// scale outer product is 2 d_w d_a (k04_operand), so a stretch's sums, and
+// the total, are golem's times 2^-21, rounded where golem's are (a power of
+// two moves no rounding; the least term that is not zero is 2^-69): the total
+// is multiplied by 2^21 once, exactly.
+constexpr int kIntBias = 0x3E400000;     // 0.1875
+constexpr float kUnscale = 2097152.0f;   // 2^21
+
+// One block's operands from LDS (a row's nibble chunk, a token's 16 bytes),
+// issued without a wait.  Written out so that the compiler sees no LDS load:
+// it would otherwise make each one wait for every load-to-LDS in flight, the
+// next stages' included.  The caller waits (lgkmcnt) before it uses them.
+template <int OFF>
+__device__ __forceinline__ void lds_read_b128(uint32_t at, v4u &r) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(r) : "v"(at), "i"(OFF));
+}
+template <int OFF>
+__device__ __forceinline__ void lds_read_b32(uint32_t at, uint32_t &r) {
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=&v"(r) : "v"(at), "i"(OFF));
+}
+template <int OFF>
+__device__ __forceinline__ void lds_read_u16(uint32_t at, uint32_t &r) {
+    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=&v"(r) : "v"(at), "i"(OFF));
 }
 
 template <int J, int N, typename F>
@@ -393,37 +377,33 @@ __device__ __forceinline__ void unroll(F &&f) {  // f(integral_constant<int, J>)
     }
 }
 
-
-// The two tile shapes of the direct-to-LDS product.  Both: a workgroup owns
-// 128 rows (two R64 tiles), a wavefront one 32x32 MFMA tile (rows 32*(w&3),
-// tokens 32*(w>>2)).
-//   TOK 64: eight wavefronts; three loads a wavefront a stage.  Slot bytes:
-//     [0, 8192) nibbles [block 4][row 128][16]
-//     [8192, 16384) int8 [block 4][half 2][token 64][16]
-//     [16384, 17408) act. scales (fp32) [block 4][token 64]
-//     [17408, 18432) weight scales (fp16) [row 128][block 4]
-//   TOK 32: four wavefronts (for batches of few tokens: an expert's share of
-//     a prompt); five loads a wavefront a stage -- two of nibbles, one of
-//     int8, two dwords of scales (the last of wavefronts 2 and 3 a dummy, so
-//     that every wavefront issues the same count).  Slot bytes:
-//     [0, 8192) nibbles [block 4][row 128][16]
-//     [8192, 12288) int8 [block 4][half 2][token 32][16]
-//     [12288, 12800) act. scales (fp32) [block 4][token 32]
-//     [12800, 13824) weight scales (fp16) [row 128][block 4]
-//     [13824, 14080) the dummy dwords
-template <int TOK>
-struct DmaShape;
-template <>
-struct DmaShape<64> {
-    static constexpr int kWaves = 8, kLoads = 3, kSlot = 18432, kOcc = 4;  // two workgroups a CU
-    static constexpr int kRing = GX_DMA_RING64;
-    static constexpr int kAct = 8192, kActScale = 16384, kWScale = 17408;
-};
-template <>
-struct DmaShape<32> {
-    static constexpr int kWaves = 4, kLoads = 5, kSlot = 14336, kOcc = 3;  // three workgroups a CU (LDS)
-    static constexpr int kRing = GX_DMA_RING32;
-    static constexpr int kAct = 8192, kActScale = 12288, kWScale = 12800, kDummy = 13824;
+// A tile shape of the product: WR x WT wavefronts of 32 rows x 32 * TT tokens.
+// Slot bytes of a stage:
+//   [0, kAct)             nibbles  [block 4][row kRows][16]
+//   [kAct, kActScale)     int8     [token kTok][16-byte piece 8], piece p of
+//                         token t in place p ^ (t & 7)
+//   [kActScale, kWScale)  act. scales (fp32) [token kTok][block 4]
+//   [kWScale, kDummy)     weight scales (fp16) [row kRows][block 4]
+//   [kDummy, + 256)       where loads go that only keep the count even
+// The activation comes in eight tokens' whole 128-byte stage rows a load
+// (eight lines; a token a lane touched 64, and its scales, a dword a lane, 64
+// more: the CU's address path, one line a clock, then set the product's
+// time), and the places' exclusive-or spreads eight tokens' same piece over
+// all banks when it is read.
+template <int TT, int WR, int WT, int RING, int OCC>
+struct GemmShape {
+    static constexpr int kTT = TT, kWR = WR, kWT = WT, kRing = RING, kOcc = OCC;
+    static constexpr int kRows = 32 * WR, kTok = 32 * TT * WT, kWaves = WR * WT, kThreads = 64 * kWaves;
+    static constexpr int kWLoads = kRows / 16 / kWaves, kALoads = kTok / 8 / kWaves;
+    static constexpr int kSLoads = (kTok / 16 + kWaves - 1) / kWaves, kDLoads = (kRows / 32 + kWaves - 1) / kWaves;
+    static constexpr int kLoads = kWLoads + kALoads + kSLoads + kDLoads;
+    static constexpr int kAct = kRows * 64, kActScale = kAct + kTok * 128, kWScale = kActScale + kTok * 16,
+                         kDummy = kWScale + kRows * 8;
+    static constexpr bool kPad = kSLoads * kWaves > kTok / 16 || kDLoads * kWaves > kRows / 32;
+    static constexpr int kSlot = kDummy + (kPad ? 256 : 0);
+    static_assert(kRows % 64 == 0 && kWLoads * kWaves * 16 == kRows && kALoads * kWaves * 8 == kTok, "whole loads");
+    static_assert((RING - 1) * kSlot + (3 * kRows * 16 > TT * 4096 ? 3 * kRows * 16 : TT * 4096) < 65536, "a read's slot and block are its immediate offset");
+    static_assert(RING * kSlot <= 160 * 1024, "the ring fits the LDS");
 };
 
 // EPI 2's epilogue (see the kernel): 4 wavefronts, wavefront rg holding
@@ -565,15 +545,15 @@ __device__ __forceinline__ void qkv_rope_epilogue(const v16f &tot, uint8_t *lds,
 }
 
 // GROUPED: blockIdx.y is an item of the expert work list (grp.work[item] =
-// {expert, first, count <= TOK, 0}; count 0 past the last item): the item's
+// {expert, first, count <= kTok, 0}; count 0 past the last item): the item's
 // tokens are units sorted[first ..], token t reading activation row
 // sorted[first + t] / act_div and writing output row sorted[first + t], all
 // against expert grp.work[item].x of the stack (matrices matrix_bytes
-// apart).  Otherwise tokens TOK * blockIdx.y .. of the batch.
+// apart).  Otherwise tokens kTok * blockIdx.y .. of the batch.
 //
-// DOTS: the same kernel, also writing every block's integer (the chain
-// difference x below) to dots[out row][n - row_start][b]; the scales are then
-// not needed, and their loads read the activation instead (in bounds).
+// DOTS: the same kernel, also writing every block's integer (x below) to
+// dots[out row][n - row_start][b]; the scales are then not needed, and their
+// loads read the activation instead (in bounds).
 //
 // EPI 1 (dense, whole matrix): the rows are gate and up interleaved by 32 (a
 // tile's rows 0..31 gate, 32..63 up, for the same 32 outputs), and the
@@ -583,48 +563,44 @@ __device__ __forceinline__ void qkv_rope_epilogue(const v16f &tot, uint8_t *lds,
 // wavefront of the gate rows, whose lane pair (l, l + 32) holds one token's
 // 32 outputs, one Q8_0 block.
 //
-// EPI 2 (dense, whole matrix, TOK 32): the rows are the query, key and value
-// heads stacked (hd = 64 or 128 rows a head, so a workgroup's 128 rows are
-// whole heads), and the product ends in qwen_qk_rope_tile_kernel's work for
-// its heads and 32 tokens, bit for bit: the sums staged in LDS by token, a
-// query or key head's RMSNormPlain (float64, left to right, a lane a token),
-// RoPE with golem's tables, fp16, the query into qr.qh and the key and value
-// into the caches -- without the [M][rows] float round trip.
-template <int TOK, bool GROUPED, bool DOTS, int EPI = 0>
-__global__ __launch_bounds__(64 * DmaShape<TOK>::kWaves, DmaShape<TOK>::kOcc) void q4_0_gemm_dma_kernel(
+// EPI 2 (dense, whole matrix, four wavefronts of rows): the rows are the
+// query, key and value heads stacked (hd = 64 or 128 rows a head, so a
+// workgroup's 128 rows are whole heads), and the product ends in
+// qwen_qk_rope_tile_kernel's work for its heads, 32 tokens at a time, bit for
+// bit: the sums staged in LDS by token, a query or key head's RMSNormPlain
+// (float64, left to right, a lane a token), RoPE with golem's tables, fp16,
+// the query into qr.qh and the key and value into the caches -- without the
+// [M][rows] float round trip.
+template <typename Sh, bool GROUPED, bool DOTS, int EPI>
+__global__ __launch_bounds__(Sh::kThreads, DOTS ? 1 : Sh::kOcc) void q4_0_gemm_kernel(
     const uint8_t *__restrict__ W, size_t plane0_bytes, int B, int DC, const int8_t *__restrict__ q,
     const float *__restrict__ scales, int K, int M, int tiles, int tile0, int row_start, int row_end,
     const float *__restrict__ bias, float *__restrict__ y, int ldy, int32_t *__restrict__ dots, Groups grp,
-    int xcd_pairs, int8_t *__restrict__ mq, float *__restrict__ ms, int32_t *__restrict__ mqs, QkvRopeArgs qr) {
-    using Sh = DmaShape<TOK>;
-    constexpr int kSlotB = Sh::kSlot;
-    // Software-pipelined blocks (one block's MFMAs ahead of the previous
-    // block's epilogue) need ~30 more registers: the 32-token form, at three
-    // workgroups a CU by its LDS, has them; the 64-token form would lose its
-    // fourth wavefront a SIMD.
-    constexpr bool kPipe = TOK == 32;
-    constexpr int kRing = Sh::kRing;
+    int xcd_cols, int8_t *__restrict__ mq, float *__restrict__ ms, int32_t *__restrict__ mqs, QkvRopeArgs qr) {
+    constexpr int kSlotB = Sh::kSlot, kRing = Sh::kRing, TT = Sh::kTT, kWaves = Sh::kWaves, kTok = Sh::kTok;
+    constexpr int kTilesWg = Sh::kRows / kTileRows;
+    constexpr int kA0 = Sh::kWLoads, kS0 = kA0 + Sh::kALoads, kD0 = kS0 + Sh::kSLoads, kLoads = Sh::kLoads;
     __shared__ __align__(16) uint8_t ring_lds[kRing * kSlotB];
     const int tid = threadIdx.x;
     const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // The workgroup's row pair bx and token group by.  With xcd_pairs > 0 the
+    // The workgroup's row group bx and token group by.  With xcd_cols > 0 the
     // grid is one-dimensional in the dispatcher's XCD order (workgroup i runs
-    // on XCD i % 8): XCD x takes row pairs [x P / 8, (x + 1) P / 8) of the P
+    // on XCD i % 8): XCD x takes row groups [x P / 8, (x + 1) P / 8) of the P
     // and every token group, token group by token group, so that its L2
     // holds its rows' weights while the tokens stream past once.  (A 2-D
-    // grid deals every XCD all row pairs: each L2 refetches the whole matrix
+    // grid deals every XCD all row groups: each L2 refetches the whole matrix
     // many times over.)
     int bx = blockIdx.x, by = blockIdx.y;
-    if (!GROUPED && xcd_pairs > 0) {
+    if (!GROUPED && xcd_cols > 0) {
         const int x = blockIdx.x & 7, local = blockIdx.x >> 3;
-        const int lo = x * xcd_pairs / 8, n = (x + 1) * xcd_pairs / 8 - lo;
-        if (local >= n * ((M + TOK - 1) / TOK))
+        const int lo = x * xcd_cols / 8, n = (x + 1) * xcd_cols / 8 - lo;
+        if (local >= n * ((M + kTok - 1) / kTok))
             return;  // this XCD's share is done: the whole workgroup
         by = local / n;
         bx = lo + (local - by * n);
     }
-    const int T0 = tile0 + 2 * bx;                // the workgroup's first R64 tile
-    const int rg = wv & 3, tg = wv >> 2;          // this wavefront's 32 rows and 32 tokens
+    const int T0 = tile0 + kTilesWg * bx;                 // the workgroup's first R64 tile
+    const int rg = wv % Sh::kWR, tg = wv / Sh::kWR;       // this wavefront's 32 rows and 32 * TT tokens
     const int li = lane & 31, g = lane >> 5;
     int first, count;
     if (GROUPED) {
@@ -635,8 +611,8 @@ __global__ __launch_bounds__(64 * DmaShape<TOK>::kWaves, DmaShape<TOK>::kOcc) vo
         W += (size_t)item.x * grp.matrix_bytes;
         first = item.y;
     } else {
-        first = by * TOK;
-        count = min(TOK, M - first);
+        first = by * kTok;
+        count = min(kTok, M - first);
     }
     // token t's activation row and output row
     auto arow = [&](int t) -> int { return GROUPED ? grp.sorted[first + t] / grp.act_div : first + t; };
@@ -649,340 +625,370 @@ __global__ __launch_bounds__(64 * DmaShape<TOK>::kWaves, DmaShape<TOK>::kOcc) vo
     // This lane's sources, fixed for the product.  Loads past the matrix, the
     // batch or the second tile read in-bounds neighbours; their values are
     // never used (weight scale 0, or not stored).
-    auto wpair_src = [&](int pidx) -> const uint8_t * {  // weight-scale pair pidx of the 256
-        const int r = pidx >> 1;
-        const int dt = min(T0 + (r >> 6), tiles - 1);
-        return W + plane0_bytes + ((size_t)dt * DC * kTileRows + (r & 63)) * kChunk + 4 * (pidx & 1);
-    };
-    const uint8_t *wsrc0, *wsrc1 = nullptr, *ssrc, *ssrc2 = nullptr;
-    const int8_t *asrc;
-    int wj, wh;
-    if constexpr (TOK == 64) {
-        wj = wv & 3, wh = wv >> 2;                // nibble load: block wj, rows 64*wh + lane
-        wsrc0 = W + ((size_t)min(T0 + wh, tiles - 1) * B * kTileRows + lane) * kChunk;
-        const int ag = wv & 1;                    // activation load: block wv >> 1, half ag, token lane
-        asrc = q + (size_t)arow(min(lane, count - 1)) * K + 16 * ag;
-        // The third load is a dword for every wavefront: waves 0..3 an
-        // activation scale (block wv, token lane), waves 4..7 a pair of
-        // weight scales (pair 64 * (wv - 4) + lane).
-        if (wv < 4)
-            ssrc = DOTS ? (const uint8_t *)(q + (size_t)arow(min(lane, count - 1)) * K)
-                        : (const uint8_t *)(scales + (size_t)arow(min(lane, count - 1)) * B);
-        else
-            ssrc = wpair_src(64 * (wv - 4) + lane);
-    } else {
-        wj = wv, wh = 0;                          // nibble loads: block wv, rows lane and 64 + lane
-        wsrc0 = W + ((size_t)min(T0, tiles - 1) * B * kTileRows + lane) * kChunk;
-        wsrc1 = W + ((size_t)min(T0 + 1, tiles - 1) * B * kTileRows + lane) * kChunk;
-        asrc = q + (size_t)arow(min(li, count - 1)) * K + 16 * g;  // block wv, half g, token li
-        // Dword A: waves 0, 1 activation scale idx = 64 wv + lane (block
-        // idx / 32, token idx % 32); waves 2, 3 weight-scale pair 64 (wv - 2)
-        // + lane.  Dword B: waves 0, 1 pair 128 + 64 wv + lane; waves 2, 3 a
-        // dummy (the pair of lane again, into the dummy dwords).
-        if (wv < 2) {
-            const int t = (64 * wv + lane) & 31;
-            ssrc = DOTS ? (const uint8_t *)(q + (size_t)arow(min(t, count - 1)) * K)
-                        : (const uint8_t *)(scales + (size_t)arow(min(t, count - 1)) * B);
-            ssrc2 = wpair_src(128 + 64 * wv + lane);
-        } else {
-            ssrc = wpair_src(64 * (wv - 2) + lane);
-            ssrc2 = ssrc;
-        }
+    // A dense product's are 32-bit offsets from its first token (a register
+    // and no address arithmetic a load), a grouped one's whole addresses.
+    using Src = std::conditional_t<GROUPED, size_t, uint32_t>;
+    const uint8_t *abase = (const uint8_t *)q + (GROUPED ? 0 : (size_t)first * K);
+    const uint8_t *sbase = DOTS ? abase : (const uint8_t *)scales + (GROUPED ? 0 : (size_t)first * B * 4);
+    Src asrc[Sh::kALoads], ssrc[Sh::kSLoads];
+    // load i of the activation: tokens 8 (wv + kWaves i) + lane / 8; of its
+    // scales: tokens 16 (wv + kWaves i) + lane / 4, block lane % 4
+#pragma unroll
+    for (int i = 0; i < Sh::kALoads; i++) {
+        const int t = min(8 * (wv + kWaves * i) + (lane >> 3), count - 1);
+        asrc[i] = (Src)(GROUPED ? arow(t) : t) * (Src)K;
     }
+#pragma unroll
+    for (int i = 0; i < Sh::kSLoads; i++) {
+        const int t = min(16 * (wv + kWaves * i) + (lane >> 2), count - 1);
+        ssrc[i] = (Src)(GROUPED ? arow(t) : t) * (Src)(DOTS ? K : 4 * B);
+    }
+    const int apiece = 16 * ((lane & 7) ^ ((lane >> 3) & 7)), sblock = lane & 3;
 
-    auto ring = [&](auto slot_tag) -> uint8_t * { return ring_lds + decltype(slot_tag)::value * kSlotB; };
-    auto issue = [&](auto slot_tag, int h) {
+    // load i of this wavefront's kLoads of a stage: nibbles, then activations, then their scales, then the weights'
+    auto issue_one = [&](auto slot_tag, auto i_tag, int h) __attribute__((always_inline)) {
+        constexpr int i = decltype(i_tag)::value;
         h = min(h, Hp - 1);  // past the last stage: the last stage again, into the free slot
-        uint8_t *slot = ring(slot_tag);
+        uint8_t *slot = ring_lds + decltype(slot_tag)::value * kSlotB;
         const int b0 = h * kStage;
-        const size_t woff = (size_t)min(b0 + wj, B - 1) * kTileRows * kChunk;
-        const size_t pair_off = (size_t)(b0 >> 3) * kTileRows * kChunk + 8 * ((b0 >> 2) & 1);
-        if constexpr (TOK == 64) {
-            __builtin_amdgcn_global_load_lds(wsrc0 + woff, (lds_ptr)(slot + (wj * 128 + 64 * wh) * 16), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(asrc + (size_t)min(b0 + (wv >> 1), B - 1) * kQ4Block,
-                                             (lds_ptr)(slot + Sh::kAct + wv * 1024), 16, 0, 0);
-            const size_t soff = wv < 4 ? (size_t)min(b0 + wv, B - 1) * 4 : pair_off;
-            __builtin_amdgcn_global_load_lds(ssrc + soff, (lds_ptr)(slot + Sh::kActScale + wv * 256), 4, 0, 0);
-        } else {
-            __builtin_amdgcn_global_load_lds(wsrc0 + woff, (lds_ptr)(slot + (wj * 128) * 16), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(wsrc1 + woff, (lds_ptr)(slot + (wj * 128 + 64) * 16), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(asrc + (size_t)min(b0 + wv, B - 1) * kQ4Block,
-                                             (lds_ptr)(slot + Sh::kAct + wv * 1024), 16, 0, 0);
-            if (wv < 2) {
-                const int blk = (64 * wv + lane) >> 5;
-                __builtin_amdgcn_global_load_lds(ssrc + (size_t)min(b0 + blk, B - 1) * 4,
-                                                 (lds_ptr)(slot + Sh::kActScale + wv * 256), 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(ssrc2 + pair_off, (lds_ptr)(slot + Sh::kWScale + 512 + wv * 256),
-                                                 4, 0, 0);
-            } else {
-                __builtin_amdgcn_global_load_lds(ssrc + pair_off, (lds_ptr)(slot + Sh::kWScale + (wv - 2) * 256),
-                                                 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(ssrc2 + pair_off, (lds_ptr)(slot + Sh::kDummy), 4, 0, 0);
-            }
+        // A uniform address (opaque, so that it stays one) plus a lane's 32-bit
+        // offset: the load takes both as they are.
+        if constexpr (i < kA0) {  // block idx % 4 of the workgroup's tile idx / 4
+            const int idx = wv + kWaves * i, blk = idx & 3, tl = idx >> 2;
+            const uint8_t *src = W + ((size_t)min(T0 + tl, tiles - 1) * B + min(b0 + blk, B - 1)) * (kTileRows * kChunk);
+            asm("" : "+s"(src));
+            src += (uint32_t)(lane * kChunk);
+            __builtin_amdgcn_global_load_lds(src, (lds_ptr)(slot + (blk * Sh::kRows + kTileRows * tl) * kChunk), 16, 0, 0);
+        } else if constexpr (i < kS0) {
+            const uint8_t *src = abase + (Src)(asrc[i - kA0] + (uint32_t)min(b0 * kQ4Block + apiece, K - 16));
+            __builtin_amdgcn_global_load_lds(src, (lds_ptr)(slot + Sh::kAct + (wv + kWaves * (i - kA0)) * 1024), 16, 0, 0);
+        } else if constexpr (i < kD0) {
+            const int idx = wv + kWaves * (i - kS0);
+            const uint8_t *src = sbase + (Src)(ssrc[i - kS0] + (uint32_t)(4 * min(b0 + sblock, B - 1)));
+            __builtin_amdgcn_global_load_lds(src, (lds_ptr)(slot + (idx < kTok / 16 ? Sh::kActScale + idx * 256 : Sh::kDummy)),
+                                             4, 0, 0);
+        } else {  // rows 32 idx + lane / 2, blocks 2 (lane % 2) ..
+            const int idx = wv + kWaves * (i - kD0), rw = min(32 * idx, Sh::kRows - 32);
+            const uint8_t *src = W + plane0_bytes +
+                                 (((size_t)min(T0 + (rw >> 6), tiles - 1) * DC + (b0 >> 3)) * kTileRows + (rw & 63)) * kChunk +
+                                 8 * ((b0 >> 2) & 1);
+            asm("" : "+s"(src));
+            src += (uint32_t)((lane >> 1) * kChunk + 4 * (lane & 1));
+            __builtin_amdgcn_global_load_lds(
+                src, (lds_ptr)(slot + (idx < Sh::kRows / 32 ? Sh::kWScale + idx * 256 : Sh::kDummy)), 4, 0, 0);
         }
     };
 
-    v16f acc, tot;
-    v16i chain;
+    // The loads of a stage spread over its 4 TT steps, kPer a step: those of step `piece`.
+    constexpr int kPer = (kLoads + kStage * TT - 1) / (kStage * TT);
+    static_assert(kPer * kStage * TT >= kLoads && kPer * TT <= kLoads, "every load has its step");
+    auto issue_step = [&](auto slot_tag, auto piece_tag, int h) __attribute__((always_inline)) {
+        constexpr int p = decltype(piece_tag)::value * kPer;
+        unroll<p, (p + kPer < kLoads ? p + kPer : kLoads)>(
+            [&](auto i_tag) __attribute__((always_inline)) { issue_one(slot_tag, i_tag, h); });
+    };
+
+    v16f acc[TT], tot[TT];
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            tot[t][e] = 0.0f;
+    v16i bias_i;
 #pragma unroll
     for (int e = 0; e < 16; e++)
-        tot[e] = 0.0f;
+        bias_i[e] = kIntBias;
     const v16f zero_f = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // This lane's LDS read addresses in slot 0 (the slot, block and half go
-    // in the reads' immediate offsets).
+    // This lane's LDS read addresses in slot 0 (the slot and block go in the
+    // reads' immediate offsets).  A block's MFMA slot k of lane half g is
+    // input 16 g + k: the low nibbles of the row's chunk for g = 0, the high
+    // ones for g = 1, against the token's piece 2 j + g of the stage.
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)ring_lds;
-    const uint32_t lds_w = lds_base + (32 * rg + li) * 16 + 8 * g;
-    const uint32_t lds_a = lds_base + Sh::kAct + (32 * tg + li) * 16 + 8 * g;
+    const uint32_t lds_w = lds_base + (32 * rg + li) * kChunk;
     const uint32_t lds_dw = lds_base + Sh::kWScale + (32 * rg + li) * 8;
-    const uint32_t lds_da = lds_base + Sh::kActScale + (32 * tg + li) * 4;
+    const uint32_t lds_da = lds_base + Sh::kActScale + (32 * TT * tg + li) * 16;
+    uint32_t lds_a[kStage];
+#pragma unroll
+    for (int j = 0; j < kStage; j++)
+        lds_a[j] = lds_base + Sh::kAct + (32 * TT * tg + li) * 128 + 16 * ((2 * j + g) ^ (li & 7));
+    const int up = g ? 0 : 4;  // brings the lane's nibble of a byte into its high half
 
-    // One stage: four blocks.  kFirst marks a stretch's first stage, whose
-    // first block starts the chain from the bias and the stretch sum from
-    // its product (x * s == fma(x, s, 0) but for the sign of a zero, which
-    // the total's 0 + P cannot show).
-    auto stage = [&](auto slot_tag, auto first_tag, int h) {
-        constexpr int kSlot = decltype(slot_tag)::value;
+    const v4h one = k0_operand(0x3C00u, g == 0), minus = k0_operand(0xB200u, g == 0);  // 1, -0.1875
+
+    // What the next block multiplies, read one block ahead.
+    uint32_t dw_n, da_n[TT];
+    v4u wq_n, bq_n[TT];
+    auto read = [&](auto slot_tag, auto j_tag) __attribute__((always_inline)) {
+        constexpr int so = decltype(slot_tag)::value * kSlotB, j = decltype(j_tag)::value;
+        lds_read_b128<so + j * Sh::kRows * kChunk>(lds_w, wq_n);
+        lds_read_u16<so + 2 * j>(lds_dw, dw_n);
+        unroll<0, TT>([&](auto t_tag) __attribute__((always_inline)) {
+            constexpr int t = decltype(t_tag)::value;
+            lds_read_b128<so + t * 4096>(lds_a[j], bq_n[t]);
+            lds_read_b32<so + t * 512 + 4 * j>(lds_da, da_n[t]);
+        });
+    };
+
+    // The reads land; their registers pass through the wait so that nothing
+    // touches them before it.
+    auto landed = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wq_n), "+v"(dw_n));
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+            asm volatile("" : "+v"(bq_n[t]), "+v"(da_n[t]));
+    };
+
+    // One stage: four blocks.  kFirst marks a stretch's first stage.  At its
+    // fourth block this wavefront holds all it needs of the stage; the next
+    // stage has landed, for every wavefront past the barrier, and this
+    // stage's slot is free: the loads of stage h + kRing go into it, spread
+    // from here to the next stage's third block.
+    auto stage = [&](auto slot_tag, auto first_tag, int h) __attribute__((always_inline)) {
+        constexpr int kSlot = decltype(slot_tag)::value, kPrev = (kSlot + kRing - 1) % kRing, kNext = (kSlot + 1) % kRing;
         constexpr bool kFirst = decltype(first_tag)::value;
-        wait_vmcnt<(kRing - 2) * Sh::kLoads>();  // stage h has landed (stages h + 1 .. may be in flight)
-        __builtin_amdgcn_s_barrier();
-        // into the slot stage h - 1 used; every wavefront is past it
-        issue(std::integral_constant<int, (kSlot + kRing - 1) % kRing>{}, h + kRing - 1);
-        constexpr int so = kSlot * kSlotB;
-        // The operands of block j + 1 are read while block j is multiplied.
-        uint2 wq_n, Bh_n, Bl_n;
-        uint32_t dwh_n;
-        float da_n;
-        auto read = [&](auto j_tag) {
-            constexpr int j = decltype(j_tag)::value;
-            lds_read_block<so + j * 2048, so + (2 * j + 1) * TOK * 16, so + 2 * j * TOK * 16, so + 2 * j,
-                           so + j * TOK * 4>(lds_w, lds_a, lds_dw, lds_da, wq_n, Bh_n, Bl_n, dwh_n, da_n);
-        };
-        read(std::integral_constant<int, 0>{});
-        // front(j): block j's operands land, block j + 1's reads go out, and
-        // block j's two MFMAs are issued; back(j): block j's chain
-        // differences and fmas.
-        v16f Sr[kStage];
-        v16i Nr[kStage];
-        auto front = [&](auto j_tag) {
+        unroll<0, kStage>([&](auto j_tag) __attribute__((always_inline)) {
             constexpr int j = decltype(j_tag)::value;
             // the previous block's work stays above this block's wait
             __builtin_amdgcn_sched_barrier(0);
-            // the reads land; the registers pass through the wait so that
-            // nothing touches them before it
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wq_n), "+v"(Bh_n), "+v"(Bl_n), "+v"(dwh_n), "+v"(da_n));
-            const uint2 wq = wq_n;
-            const v4i Bv = {(int)Bh_n.x, (int)Bh_n.y, (int)Bl_n.x, (int)Bl_n.y};
-            const uint32_t dwh = dwh_n;
-            const float da = da_n;
+            landed();
+            if constexpr (j == kStage - 1) {
+                wait_vmcnt<(kRing - 2) * kLoads>();
+                __builtin_amdgcn_s_barrier();
+            }
+            const v4h dwop = k04_operand(dw_n);
+            v4i A;  // 16 (n - 8) in every byte
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                A[i] = (int)(((wq_n[i] << up) & 0xF0F0F0F0u) ^ 0x80808080u);
+            v4u bq[TT];
+            uint32_t dah[TT];
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                bq[t] = bq_n[t];
+                dah[t] = half2_bits_rtz(__uint_as_float(da_n[t]));
+            }
             if constexpr (j + 1 < kStage)
-                read(std::integral_constant<int, j + 1>{});
-            // The scale outer product goes to the matrix core first: it does
-            // not wait for the chain, and the integer MFMA queues behind it
-            // while the nibbles are widened.  (Issued after the integer MFMA,
-            // the compiler put the first chain difference ahead of it, so
-            // the scales waited for the integers: two MFMA latencies a
-            // block.)
-            // a block past the row has weight scale 0 (the padding is zero):
-            // fma(x, 0, acc) == acc
-            Sr[j] = __builtin_amdgcn_mfma_f32_32x32x8f16(k04_operand(dwh), k04_operand(half2_bits_rtz(da)), zero_f, 0,
-                                                          0, 0);
-            // 16 (n - 8) in every byte: the high nibbles in place, the low
-            // ones shifted up, the top bit flipped
-            v4i A;
-            A.x = (int)((wq.x & 0xF0F0F0F0u) ^ 0x80808080u);
-            A.y = (int)((wq.y & 0xF0F0F0F0u) ^ 0x80808080u);
-            A.z = (int)(((wq.x << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
-            A.w = (int)(((wq.y << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
-            v16i prev;
-            if constexpr (kFirst && j == 0) {
-                // written afresh each stretch (a resident copy would cost 16
-                // registers and a wavefront per SIMD)
+                read(slot_tag, std::integral_constant<int, j + 1>{});
+            else
+                read(std::integral_constant<int, kNext>{}, std::integral_constant<int, 0>{});
+            unroll<0, TT>([&](auto t_tag) __attribute__((always_inline)) {
+                constexpr int t = decltype(t_tag)::value;
+                // a block past the row has weight scale 0 (the padding is zero):
+                // fma(x, 0, acc) == acc
+                const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, __builtin_bit_cast(v4i, bq[t]), bias_i, 0, 0, 0);
+                const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(dwop, k04_operand(dah[t]), zero_f, 0, 0, 0);
+                const v16f X =
+                    __builtin_amdgcn_mfma_f32_32x32x8f16(one, minus, __builtin_bit_cast(v16f, D), 0, 0, 0);  // isum * 2^-22
+                constexpr int piece = ((j + 1) % kStage) * TT + t;  // of the stage being loaded
+                if constexpr (j == kStage - 1)
+                    issue_step(slot_tag, std::integral_constant<int, piece>{}, h + kRing);
+                else
+                    issue_step(std::integral_constant<int, kPrev>{}, std::integral_constant<int, piece>{}, h - 1 + kRing);
+                __builtin_amdgcn_sched_barrier(0);
+                // a stretch's first block takes the product for the sum (x *
+                // s == fma(x, s, 0) but for the sign of a zero, which the
+                // total's 0 + P cannot show); its eighth adds it to the total
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    acc[t][e] = kFirst && j == 0 ? X[e] * S[e] : fmaf(X[e], S[e], acc[t][e]);
+                if constexpr (!kFirst && j == kStage - 1) {
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        tot[t][e] = tot[t][e] + acc[t][e];
+                }
+                // the sums are complete here, not sunk past the next barrier
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    int bias;
-                    asm volatile("v_mov_b32 %0, %1" : "=v"(bias) : "i"(kChainBias));
-                    prev[e] = bias;
+                    if constexpr (!kFirst && j == kStage - 1)
+                        asm volatile("" : "+v"(tot[t][e]));
+                    else
+                        asm volatile("" : "+v"(acc[t][e]));
                 }
-            } else if constexpr (j == 0) {
-                prev = chain;
-            } else {
-                prev = Nr[j - 1];
-            }
-            Nr[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, Bv, prev, 0, 0, 0);
-        };
-        auto back = [&](auto j_tag) {
-            constexpr int j = decltype(j_tag)::value;
-            constexpr bool start = kFirst && j == 0;
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                // half the block's isum, exactly (a stretch's first block
-                // subtracts the bias as a literal: its MFMA then runs in
-                // place, with no copy of the bias kept for the difference)
-                int pb;
-                if constexpr (start)
-                    pb = kChainBias;
-                else if constexpr (j == 0)
-                    pb = chain[e];
-                else
-                    pb = Nr[j - 1][e];
-                const float x = __int_as_float(Nr[j][e]) - __int_as_float(pb);
-                acc[e] = start ? x * Sr[j][e] : fmaf(x, Sr[j][e], acc[e]);
                 if constexpr (DOTS) {
-                    const int b = h * kStage + j, tt = 32 * tg + li;
-                    const int n = T0 * kTileRows + 32 * rg + 8 * (e >> 2) + 4 * g + (e & 3);
-                    if (b < B && tt < count && n >= row_start && n < row_end)
-                        dots[((size_t)orow(tt) * (row_end - row_start) + (n - row_start)) * B + b] = (int)(2.0f * x);
-                }
-            }
-        };
-        if constexpr (kPipe) {
-            // block j + 1's MFMAs go out before block j's differences, which
-            // then run while the matrix core works on them
-            front(std::integral_constant<int, 0>{});
-            unroll<0, kStage>([&](auto j_tag) {
-                constexpr int j = decltype(j_tag)::value;
-                if constexpr (j + 1 < kStage)
-                    front(std::integral_constant<int, j + 1>{});
-                __builtin_amdgcn_sched_barrier(0);
-                back(j_tag);
-            });
-        } else {
-            unroll<0, kStage>([&](auto j_tag) {
-                front(j_tag);
-                __builtin_amdgcn_sched_barrier(0);
-                back(j_tag);
-            });
-        }
-        chain = Nr[kStage - 1];
-        // the stage's sums are complete here, not sunk past the next barrier
+                    const int tt = 32 * (TT * tg + t) + li, b = h * kStage + j;
 #pragma unroll
-        for (int e = 0; e < 16; e++)
-            asm volatile("" : "+v"(acc[e]));
+                    for (int e = 0; e < 16; e++) {
+                        const int n = T0 * kTileRows + 32 * rg + 8 * (e >> 2) + 4 * g + (e & 3);
+                        if (b < B && tt < count && n >= row_start && n < row_end)
+                            dots[((size_t)orow(tt) * (row_end - row_start) + (n - row_start)) * B + b] =
+                                (int)(X[e] * 4194304.0f);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
     };
 
-    auto fold = [&]() {  // a stretch is two stages
-#pragma unroll
-        for (int e = 0; e < 16; e++)
-            tot[e] = tot[e] + acc[e];
-    };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    using S2 = std::integral_constant<int, 2>;
-    if constexpr (kRing == 3) {
-        issue(S0{}, 0);
-        issue(S1{}, 1);
+    // Stages 0 .. kRing - 2 whole, and the pieces of stage kRing - 1 that
+    // come before a stage's first block (the rest follow in stage 0).
+    unroll<0, kRing - 1>([&](auto n_tag) __attribute__((always_inline)) {
+        unroll<0, kLoads>([&](auto i_tag) __attribute__((always_inline)) { issue_one(n_tag, i_tag, decltype(n_tag)::value); });
+    });
+    unroll<0, TT>([&](auto t_tag) __attribute__((always_inline)) {
+        issue_step(std::integral_constant<int, kRing - 1>{}, t_tag, kRing - 1);
+    });
+    wait_vmcnt<(kRing - 2) * kLoads + kPer * TT>();  // stage 0 has landed
+    __builtin_amdgcn_s_barrier();
+    read(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+    using F = std::true_type;
+    using N = std::false_type;
+    if constexpr (kRing == 2) {
+        for (int h = 0; h < Hp; h += 2) {
+            stage(std::integral_constant<int, 0>{}, F{}, h);
+            stage(std::integral_constant<int, 1>{}, N{}, h + 1);
+        }
+    } else if constexpr (kRing == 3) {
         for (int h = 0;; h += 6) {  // three stretches: the ring comes round to slot 0
-            stage(S0{}, std::true_type{}, h);
-            stage(S1{}, std::false_type{}, h + 1);
-            fold();
+            stage(std::integral_constant<int, 0>{}, F{}, h);
+            stage(std::integral_constant<int, 1>{}, N{}, h + 1);
             if (h + 2 >= Hp)
                 break;
-            stage(S2{}, std::true_type{}, h + 2);
-            stage(S0{}, std::false_type{}, h + 3);
-            fold();
+            stage(std::integral_constant<int, 2>{}, F{}, h + 2);
+            stage(std::integral_constant<int, 0>{}, N{}, h + 3);
             if (h + 4 >= Hp)
                 break;
-            stage(S1{}, std::true_type{}, h + 4);
-            stage(S2{}, std::false_type{}, h + 5);
-            fold();
+            stage(std::integral_constant<int, 1>{}, F{}, h + 4);
+            stage(std::integral_constant<int, 2>{}, N{}, h + 5);
             if (h + 6 >= Hp)
                 break;
         }
     } else {
-        using S3 = std::integral_constant<int, 3>;
-        issue(S0{}, 0);
-        issue(S1{}, 1);
-        issue(S2{}, 2);
+        static_assert(kRing == 4, "rings of two to four slots");
         for (int h = 0;; h += 4) {  // two stretches: the ring comes round to slot 0
-            stage(S0{}, std::true_type{}, h);
-            stage(S1{}, std::false_type{}, h + 1);
-            fold();
+            stage(std::integral_constant<int, 0>{}, F{}, h);
+            stage(std::integral_constant<int, 1>{}, N{}, h + 1);
             if (h + 2 >= Hp)
                 break;
-            stage(S2{}, std::true_type{}, h + 2);
-            stage(S3{}, std::false_type{}, h + 3);
-            fold();
+            stage(std::integral_constant<int, 2>{}, F{}, h + 2);
+            stage(std::integral_constant<int, 3>{}, N{}, h + 3);
             if (h + 4 >= Hp)
                 break;
         }
     }
+    landed();         // the last block's reads ahead: into registers that are free from here
     wait_vmcnt<0>();  // the trailing loads land before the workgroup ends
-    const int t = 32 * tg + li;
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            tot[t][e] = tot[t][e] * kUnscale;
+    // the lane again, so that no register holds it through the loop
+    const int elane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), eli = elane & 31, eg = elane >> 5;
     if constexpr (EPI == 1) {
         __syncthreads();  // every wavefront is past its last operand reads
-        float *xch = (float *)ring_lds;  // [wavefront pair][lane][17]
+        float *xch = (float *)ring_lds;  // [wavefront pair][token tile][lane][17]
         const int pair = wv >> 1;
         if (rg & 1) {
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                xch[(pair * 64 + lane) * 17 + e] = tot[e];
+            for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    xch[((pair * TT + tt) * 64 + 32 * eg + eli) * 17 + e] = tot[tt][e];
         }
         __syncthreads();
         const int tile = T0 + (rg >> 1);
         if (!(rg & 1) && tile * kTileRows < row_end) {
-            const int F = row_end >> 1;  // outputs a token
-            float v[16];
+            const int F2 = row_end >> 1;  // outputs a token
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const float gt = tot[e], u = xch[(pair * 64 + lane) * 17 + e];
-                const float ex = ggml_expf(-gt);
-                const float den = 1.0f + ex;
-                const float sl = gt / den;
-                v[e] = sl * u;
-            }
-            float peak = fabsf(v[0]);
-#pragma unroll
-            for (int e = 1; e < 16; e++)
-                peak = fmaxf(peak, fabsf(v[e]));
-            peak = fmaxf(peak, __shfl_xor(peak, 32, 64));  // the token's other 16 outputs
-            int32_t n[16];
-            float stored = 0.0f;
-            if (peak == 0.0f) {
-#pragma unroll
-                for (int e = 0; e < 16; e++)
-                    n[e] = 0;
-            } else {
-                const float scale = __fdiv_rn(peak, 127.0f);
-                const float inverse = __fdiv_rn(127.0f, peak);
-                stored = half_bits_to_float(float_to_half_bits(scale));
+            for (int tt = 0; tt < TT; tt++) {
+                const int t = 32 * (TT * tg + tt) + eli;
+                float v[16];
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    const int32_t k = nearest_int(v[e] * inverse);
-                    n[e] = k > 127 ? 127 : (k < -128 ? -128 : k);
+                    const float gt = tot[tt][e], u = xch[((pair * TT + tt) * 64 + 32 * eg + eli) * 17 + e];
+                    const float ex = ggml_expf(-gt);
+                    const float den = 1.0f + ex;
+                    const float sl = gt / den;
+                    v[e] = sl * u;
                 }
-            }
-            int32_t sum = 0;
+                float peak = fabsf(v[0]);
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                sum += n[e];
-            sum += __shfl_xor(sum, 32, 64);
-            if (t < count) {
-                const int row = orow(t);
-                // element e is output 8 (e / 4) + 4 g + e % 4 of the tile's 32
+                for (int e = 1; e < 16; e++)
+                    peak = fmaxf(peak, fabsf(v[e]));
+                peak = fmaxf(peak, __shfl_xor(peak, 32, 64));  // the token's other 16 outputs
+                int32_t n[16];
+                float stored = 0.0f;
+                if (peak == 0.0f) {
 #pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) {
-                    const uint32_t w = (uint32_t)(n[4 * e4] & 0xFF) | ((uint32_t)(n[4 * e4 + 1] & 0xFF) << 8) |
-                                       ((uint32_t)(n[4 * e4 + 2] & 0xFF) << 16) |
-                                       ((uint32_t)(n[4 * e4 + 3] & 0xFF) << 24);
-                    *(uint32_t *)(mq + (size_t)row * F + tile * 32 + 8 * e4 + 4 * g) = w;
+                    for (int e = 0; e < 16; e++)
+                        n[e] = 0;
+                } else {
+                    const float scale = __fdiv_rn(peak, 127.0f);
+                    const float inverse = __fdiv_rn(127.0f, peak);
+                    stored = half_bits_to_float(float_to_half_bits(scale));
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const int32_t k = nearest_int(v[e] * inverse);
+                        n[e] = k > 127 ? 127 : (k < -128 ? -128 : k);
+                    }
                 }
-                if (g == 0) {
-                    ms[(size_t)row * (F >> 5) + tile] = stored;
-                    mqs[(size_t)row * (F >> 5) + tile] = sum;
+                int32_t sum = 0;
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    sum += n[e];
+                sum += __shfl_xor(sum, 32, 64);
+                if (t < count) {
+                    const int row = orow(t);
+                    // element e is output 8 (e / 4) + 4 eg + e % 4 of the tile's 32
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; e4++) {
+                        const uint32_t w = (uint32_t)(n[4 * e4] & 0xFF) | ((uint32_t)(n[4 * e4 + 1] & 0xFF) << 8) |
+                                           ((uint32_t)(n[4 * e4 + 2] & 0xFF) << 16) |
+                                           ((uint32_t)(n[4 * e4 + 3] & 0xFF) << 24);
+                        *(uint32_t *)(mq + (size_t)row * F2 + tile * 32 + 8 * e4 + 4 * eg) = w;
+                    }
+                    if (eg == 0) {
+                        ms[(size_t)row * (F2 >> 5) + tile] = stored;
+                        mqs[(size_t)row * (F2 >> 5) + tile] = sum;
+                    }
                 }
             }
         }
     } else if constexpr (EPI == 2) {
-        static_assert(TOK == 32 && !GROUPED && !DOTS, "the Q|K|V epilogue is a dense 32-token form");
-        qkv_rope_epilogue(tot, ring_lds, qr, T0, rg, li, g, first, count);
-    } else if (!DOTS && t < count) {
-        float *yr = y + (size_t)orow(t) * ldy;
-        const int nb = T0 * kTileRows + 32 * rg;  // the wavefront's first row
+        static_assert(Sh::kWR == 4 && Sh::kWT == 1 && !GROUPED && !DOTS, "the Q|K|V epilogue: 128 rows, 256 threads");
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const int n = nb + 8 * (e >> 2) + 4 * g + (e & 3);
-            if (n >= row_start && n < row_end)
-                yr[n] = bias ? tot[e] + bias[n] : tot[e];
+        for (int tt = 0; tt < TT; tt++)
+            if (32 * tt < count)
+                qkv_rope_epilogue(tot[tt], ring_lds, qr, T0, rg, li, g, first + 32 * tt, min(32, count - 32 * tt));
+    } else if constexpr (!DOTS) {
+        const int nb = T0 * kTileRows + 32 * rg;  // the wavefront's first row
+        // four rows a store where the output takes 16-byte stores
+        const bool wide = (ldy & 3) == 0 && ((uintptr_t)y & 15) == 0;
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++) {
+            const int t = 32 * (TT * tg + tt) + eli;
+            if (t >= count)
+                continue;
+            float *yr = y + (size_t)orow(t) * ldy;
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) {
+                const int n0 = nb + 8 * e4 + 4 * eg;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    v[e] = tot[tt][4 * e4 + e];
+                if (n0 >= row_start && n0 + 4 <= row_end) {
+                    if (bias) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            v[e] = v[e] + bias[n0 + e];
+                    }
+                    if (wide) {
+                        *(float4 *)(yr + n0) = make_float4(v[0], v[1], v[2], v[3]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            yr[n0 + e] = v[e];
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int n = n0 + e;
+                        if (n >= row_start && n < row_end)
+                            yr[n] = bias ? v[e] + bias[n] : v[e];
+                    }
+                }
+            }
         }
     }
 }
@@ -990,81 +996,83 @@ __global__ __launch_bounds__(64 * DmaShape<TOK>::kWaves, DmaShape<TOK>::kOcc) vo
 }  // namespace
 
 namespace {
-// The dense product's grid and launch (EPI 0: y = the product; EPI 1: the
-// SwiGLU + Q8_0 epilogue into mq / ms / mqs).
-template <int EPI>
-int launch_dense(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8_t *q, const float *scales, int M,
+// Three wavefronts a SIMD each (twelve a CU, in three to six workgroups).  128
+// x 64: two token tiles a wavefront share its widened weights; 168 registers
+// and a ring of two.  64 x 64 and 128 x 32: one tile a wavefront.
+using Shape128x64 = GemmShape<2, 4, 1, 2, 3>;
+using Shape64x64 = GemmShape<1, 2, 2, 2, 3>;
+using Shape128x32 = GemmShape<1, 4, 1, 3, 3>;
+
+template <typename Sh, bool DD, int EPI>
+int launch_shape(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8_t *q, const float *scales, int M,
                  int row_start, int row_end, const float *bias, float *y, int ldy, int32_t *dots, int8_t *mq,
-                 float *ms, int32_t *mqs) {
+                 float *ms, int32_t *mqs, const QkvRopeArgs &qr) {
+    constexpr int kTiles = Sh::kRows / kTileRows;
     // the widened weights are signed: no recentring term, so no qsum
     const int tile0 = row_start / kTileRows;
     const int tiles = (row_end + kTileRows - 1) / kTileRows - tile0;
     const Groups none{nullptr, nullptr, 1, 0};
-    const int pairs = (tiles + 1) / 2;
-    // Up to 1024 tokens, 32-token workgroups: twice as many of them to fill
-    // the CUs (config 2's 9728 x 2560 in a graph over rotating copies: M = 64
-    // 25.0 -> 20.1 us, M = 512 62.0 -> 56.1 us; M = 2048 195 against 198 us
-    // keeps 64), unless the 64-token form has a thousand workgroups anyway
-    // (config 3's Gate|Up, 19456 rows, at a 512-token prompt: the prefill
-    // 9.93 -> 9.80 ms).  Between 256 and 512 of them, though, some CUs take
-    // two 32-token workgroups to the others' one, where the 64-token form
-    // fits in one round (config 3's O and Down, 2560 rows, at a 512-token
-    // prompt: 35.1 -> 33.1 and 71.0 -> 63.6 us).  The per-token arithmetic
-    // is the same either way.
-    const int w32 = pairs * ((M + 31) / 32);
-    const int tok = (M <= 1024 && pairs * ((M + kDmaTok - 1) / kDmaTok) < 1000 && (w32 <= 256 || w32 > 512))
-                        ? 32
-                        : kDmaTok;
-    const int groups = (M + tok - 1) / tok;
-    // XCD order for matrices of at least eight row pairs (every XCD some).
-    const int xp = pairs >= 8 ? pairs : 0;
-    const dim3 grid = xp ? dim3((unsigned)(8 * ((pairs + 7) / 8) * groups)) : dim3((unsigned)pairs, (unsigned)groups);
-#define GX_DMA_LAUNCH(TK, NT, DD)                                                                                   \
-    q4_0_gemm_dma_kernel<TK, false, DD, EPI><<<grid, NT, 0, ctx->stream>>>(                                         \
-        mat, w->plane0_bytes, w->blocks, w->dchunks, q, scales, w->cols, M, w->tiles, tile0, row_start, row_end,     \
-        bias, y, ldy, DD ? dots : nullptr, none, xp, mq, ms, mqs, QkvRopeArgs{})
-    if constexpr (EPI == 1) {
-        if (tok == 32)
-            GX_DMA_LAUNCH(32, 256, false);
-        else
-            GX_DMA_LAUNCH(64, 512, false);
-    } else {
-        if (tok == 32 && dots)
-            GX_DMA_LAUNCH(32, 256, true);
-        else if (tok == 32)
-            GX_DMA_LAUNCH(32, 256, false);
-        else if (dots)
-            GX_DMA_LAUNCH(64, 512, true);
-        else
-            GX_DMA_LAUNCH(64, 512, false);
-    }
-#undef GX_DMA_LAUNCH
+    const int cols = (tiles + kTiles - 1) / kTiles;
+    const int groups = (M + Sh::kTok - 1) / Sh::kTok;
+    // XCD order for matrices of at least eight row groups (every XCD some).
+    const int xc = cols >= 8 ? cols : 0;
+    const dim3 grid = xc ? dim3((unsigned)(8 * ((cols + 7) / 8) * groups)) : dim3((unsigned)cols, (unsigned)groups);
+    q4_0_gemm_kernel<Sh, false, DD, EPI><<<grid, Sh::kThreads, 0, ctx->stream>>>(
+        mat, w->plane0_bytes, w->blocks, w->dchunks, q, scales, w->cols, M, w->tiles, tile0, row_start, row_end, bias,
+        y, ldy, dots, none, xc, mq, ms, mqs, qr);
     return check_launch("q4_0_gemm");
+}
+
+// The shape of a dense product: 128 x 64 where three of its workgroups fall to
+// every CU (a CU holds three), one round whole or more; fewer leave CUs
+// part empty for the length of a whole tile, and 64 x 64 with twice as many
+// wavefronts ends sooner.  9728 x 2560 (us, 128 x 64 / 64 x 64): M = 2048 126
+// / 137, 1000 65 / 72, 500 38.7 / 38.0, 300 27.6 / 24.2; 2560 x 4096 at 1500
+// (480 workgroups) 55.8 / 46.6; 6144 x 2560 at 1500 (1152) 64.1 / 66.9.  Up
+// to 32 tokens half of a 64-token tile would be empty: 128 x 32 (19456 x 2560
+// with SwiGLU at 32: 15.0 against 17.9), as the Q|K|V epilogue has for its
+// small form, whose heads need 128 rows.
+template <int EPI>
+int launch_dense(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8_t *q, const float *scales, int M,
+                 int row_start, int row_end, const float *bias, float *y, int ldy, int32_t *dots, int8_t *mq,
+                 float *ms, int32_t *mqs, const QkvRopeArgs &qr) {
+    const int tiles = (row_end + kTileRows - 1) / kTileRows - row_start / kTileRows;
+    const size_t big = (size_t)((tiles + 1) / 2) * ((M + 63) / 64);
+#define GX_SHAPE(SH)                                                                                                 \
+    do {                                                                                                             \
+        if (EPI == 0 && dots)                                                                                        \
+            return launch_shape<SH, EPI == 0, EPI>(ctx, w, mat, q, scales, M, row_start, row_end, bias, y, ldy,     \
+                                                   dots, mq, ms, mqs, qr);                                          \
+        return launch_shape<SH, false, EPI>(ctx, w, mat, q, scales, M, row_start, row_end, bias, y, ldy, nullptr,   \
+                                            mq, ms, mqs, qr);                                                       \
+    } while (0)
+    if (big >= 3 * (size_t)ctx->cu_count)
+        GX_SHAPE(Shape128x64);
+    if constexpr (EPI != 2) {
+        if (M > 32)
+            GX_SHAPE(Shape64x64);
+    }
+    GX_SHAPE(Shape128x32);
+#undef GX_SHAPE
 }
 }  // namespace
 
 int launch_q4_0_gemm(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8_t *q, const float *scales,
                      int M, int row_start, int row_end, const float *bias, float *y, int ldy, int32_t *dots) {
     return launch_dense<0>(ctx, w, mat, q, scales, M, row_start, row_end, bias, y, ldy, dots, nullptr, nullptr,
-                           nullptr);
+                           nullptr, QkvRopeArgs{});
 }
 
 int launch_q4_0_gemm_swiglu(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *scales, int M,
                             int8_t *mq, float *ms, int32_t *mqs) {
-    return launch_dense<1>(ctx, w, w->dev, q, scales, M, 0, w->rows, nullptr, nullptr, 0, nullptr, mq, ms, mqs);
+    return launch_dense<1>(ctx, w, w->dev, q, scales, M, 0, w->rows, nullptr, nullptr, 0, nullptr, mq, ms, mqs,
+                           QkvRopeArgs{});
 }
 
 int launch_q4_0_gemm_qkv_rope(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *scales, int M,
                               const QkvRopeArgs &a) {
-    // the 32-token form always (its epilogue's shape), in XCD order
-    const int pairs = (w->tiles + 1) / 2, groups = (M + 31) / 32;
-    const Groups none{nullptr, nullptr, 1, 0};
-    const int xp = pairs >= 8 ? pairs : 0;
-    const dim3 grid = xp ? dim3((unsigned)(8 * ((pairs + 7) / 8) * groups)) : dim3((unsigned)pairs, (unsigned)groups);
-    q4_0_gemm_dma_kernel<32, false, false, 2><<<grid, 256, 0, ctx->stream>>>(
-        w->dev, w->plane0_bytes, w->blocks, w->dchunks, q, scales, w->cols, M, w->tiles, 0, 0, w->rows, nullptr,
-        nullptr, 0, nullptr, none, xp, nullptr, nullptr, nullptr, a);
-    return check_launch("q4_0_gemm qkv_rope");
+    return launch_dense<2>(ctx, w, w->dev, q, scales, M, 0, w->rows, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
+                           nullptr, a);
 }
 
 int launch_q4_0_gemm_grouped(gx_ctx *ctx, const gx_weight *w, const int32_t *work, int max_items,
@@ -1074,11 +1082,11 @@ int launch_q4_0_gemm_grouped(gx_ctx *ctx, const gx_weight *w, const int32_t *wor
     const dim3 grid((unsigned)((w->tiles + 1) / 2), (unsigned)max_items);
     const Groups grp{work, sorted, act_div, w->matrix_bytes};
     if (dots)
-        q4_0_gemm_dma_kernel<32, true, true><<<grid, 256, 0, ctx->stream>>>(
+        q4_0_gemm_kernel<Shape128x32, true, true, 0><<<grid, Shape128x32::kThreads, 0, ctx->stream>>>(
             w->dev, w->plane0_bytes, w->blocks, w->dchunks, q, scales, w->cols, 0, w->tiles, 0, 0, w->rows, nullptr,
             y, ldy, dots, grp, 0, nullptr, nullptr, nullptr, QkvRopeArgs{});
     else
-        q4_0_gemm_dma_kernel<32, true, false><<<grid, 256, 0, ctx->stream>>>(
+        q4_0_gemm_kernel<Shape128x32, true, false, 0><<<grid, Shape128x32::kThreads, 0, ctx->stream>>>(
             w->dev, w->plane0_bytes, w->blocks, w->dchunks, q, scales, w->cols, 0, w->tiles, 0, 0, w->rows, nullptr,
             y, ldy, nullptr, grp, 0, nullptr, nullptr, nullptr, QkvRopeArgs{});
     return check_launch("q4_0_gemm_grouped");
