@@ -957,13 +957,13 @@ static int attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_h
     GX_CHECK(!slots || nslots > 0, "gx: %d slots", nslots);
     if (M == 0)
         return ok();
-    const size_t need = gx::qwen_attention_workspace(M, heads, max_pos);
+    const size_t need = gx::qwen_attention_workspace_least(M, heads, max_pos);
     GX_CHECK(workspace_bytes >= need, "gx: the workspace holds %zu bytes, %zu needed", workspace_bytes, need);
     // llama.cpp's 1/sqrt(head_dim), taken in float64 and rounded (qwen/attention.go:90-93)
     const float scale = (float)(1.0 / sqrt((double)head_dim));
     if (int rc = gx::launch_qwen_attention(ctx, qh, M, heads, kv_heads, head_dim, max_pos, positions, kcache, vcache,
-                                           context, scale, q, scales, qsum, (uint8_t *)workspace, slots,
-                                           nslots, parallel, nullptr))
+                                           context, scale, q, scales, qsum, (uint8_t *)workspace,
+                                           workspace_bytes, slots, nslots, parallel, nullptr))
         return rc;
     return ok();
 }
@@ -993,7 +993,7 @@ int gx_qwen_attention_heads(gx_ctx *ctx, const uint16_t *qh, int M, int heads, i
     GX_CHECK(((uintptr_t)vcache & 15) == 0, "gx: the value cache must be 16-byte aligned");
     const float scale = (float)(1.0 / sqrt((double)head_dim));
     if (int rc = gx::launch_qwen_attention(ctx, qh, M, heads, kv_heads, head_dim, max_pos, positions, kcache, vcache,
-                                           context, scale, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 1, out))
+                                           context, scale, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 0, 1, out))
         return rc;
     return ok();
 }

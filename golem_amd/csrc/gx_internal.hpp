@@ -171,7 +171,17 @@ int launch_qwen_qk_rope(gx_ctx *ctx, const float *qkv, int ldqkv, int M, int hea
                         const int32_t *positions, const float *q_norm, const float *k_norm, const float *rope_cos,
                         const float *rope_sin, float eps, uint16_t *qh, uint16_t *kcache, uint16_t *vcache,
                         int context, const int32_t *slots, int nslots);
-size_t qwen_attention_workspace(int M, int heads, int max_pos);
+size_t qwen_attention_workspace(int M, int heads, int max_pos);       // what the calls' callers allocate
+size_t qwen_attention_workspace_least(int M, int heads, int max_pos); // what a call cannot do without
+bool attn_prompt_long_fits(int hd, int limit);
+int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
+                            const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
+                            float scale, int8_t *q, float *scales, int32_t *qsum);
+size_t attn_split_workspace(int M, int heads, int S);
+int launch_attn_split(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
+                      const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
+                      float scale, int8_t *q, float *scales, int32_t *qsum, float *sc, float *small, float *runs,
+                      const int32_t *slots, int nslots);
 int launch_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int M, int heads, int kv_heads, int hd,
                                int max_pos, const int32_t *positions, const float *q_norm, const float *k_norm,
                                const float *rope_cos, const float *rope_sin, float eps, uint16_t *kcache,
@@ -180,7 +190,7 @@ int launch_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int M, 
 int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int max_pos,
                           const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                           float scale, int8_t *q, float *scales, int32_t *qsum, uint8_t *workspace,
-                          const int32_t *slots, int nslots, int parallel, float *heads_f);
+                          size_t workspace_bytes, const int32_t *slots, int nslots, int parallel, float *heads_f);
 int launch_qwen_swiglu_quant(gx_ctx *ctx, const float *gu, int ldgu, int M, int ffn, int group, int8_t *q,
                              float *scales, int32_t *qsum);
 int launch_argmax(gx_ctx *ctx, const float *x, int ldx, int M, int n, int32_t *out, int32_t *history,

@@ -2170,17 +2170,25 @@ int launch_qwen_qk_rope(gx_ctx *ctx, const float *qkv, int ldqkv, int M, int hea
     return check_launch("qwen_qk_rope");
 }
 
-size_t qwen_attention_workspace(int M, int heads, int max_pos) {
+size_t qwen_attention_workspace_least(int M, int heads, int max_pos) {
     const size_t S = ((size_t)max_pos + kTile) / kTile * kTile;
     const size_t rows = (size_t)M * heads;
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     return up(rows * S * sizeof(float)) + up(rows * S * sizeof(uint16_t));
 }
 
+// Past the one-workgroup decode form's prefixes, the runs of the split form
+// too (a caller with the least alone gets the serial passes).
+size_t qwen_attention_workspace(int M, int heads, int max_pos) {
+    const int S = (max_pos + kTile) / kTile * kTile;
+    return qwen_attention_workspace_least(M, heads, max_pos) +
+           (max_pos < kDecodeMax ? 0 : attn_split_workspace(M, heads, S));
+}
+
 int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int max_pos,
                           const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                           float scale, int8_t *q, float *scales, int32_t *qsum, uint8_t *workspace,
-                          const int32_t *slots, int nslots, int parallel, float *heads_f) {
+                          size_t workspace_bytes, const int32_t *slots, int nslots, int parallel, float *heads_f) {
     const int G = heads / kv_heads;
     GX_CHECK(hd == 32 || hd == 64 || hd == 96 || hd == 128, "gx: attention supports head widths 32, 64, 96 and 128");
     GX_CHECK(G == 1 || G == 2 || G == 4 || G == 8, "gx: %d query heads per key-value head unsupported", G);
@@ -2196,10 +2204,20 @@ int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int
     if (parallel && (M <= 4 || slots) && limit <= kDecodeMax)
         return launch_par<false>(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context, scale,
                                  q, scales, qsum, slots, nslots, QkRope{}, heads_f);
+    // Longer prefixes: the same order, the positions spread over the chip.
+    // (One position of 32 heads at 3,000: 104 us in the serial passes.)
+    if (parallel && (M <= 4 || slots) && !heads_f && workspace_bytes >= qwen_attention_workspace(M, heads, max_pos))
+        return launch_attn_split(ctx, qh, M, heads, kv_heads, hd, limit, S, positions, kcache, vcache, context, scale,
+                                 q, scales, qsum, sc, (float *)prob,
+                                 (float *)(workspace + qwen_attention_workspace_least(M, heads, max_pos)), slots,
+                                 nslots);
     // A prompt of one conversation in the parallel order: the matrix cores.
     if (parallel && !slots && limit <= kPmMax)
         return launch_prompt_mfma(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context, scale,
                                   q, scales, qsum, heads_f);
+    if (parallel && !slots && M > 4 && attn_prompt_long_fits(hd, limit))
+        return launch_attn_prompt_long(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context,
+                                       scale, q, scales, qsum);
     if ((M <= 4 || slots) && limit <= kDecodeMax) {
 // One query head per workgroup when that fills at most two workgroups per CU
 // (128 workgroups for config 3's decode rather than 32): the scores,

@@ -432,7 +432,8 @@ int gx_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int heads, 
 
 /* gx_qwen_attention and gx_qwen_rope_attention with their two serial sums
  * taken in parallel, for decode steps (M <= 4 positions of one conversation,
- * or one position per conversation with slots; prefixes of at most 768):
+ * or one position per conversation with slots; the one-kernel form takes
+ * prefixes of at most 768, gx_qwen_attention_parallel any):
  * SoftmaxInPlace's total (nn/ops.go:59-73) as a tree over the positions, and
  * each head element's Axpy over the positions (nn/kernel.go:221-233) as 16
  * runs of consecutive positions added in run order.  The scores, maximum,
@@ -445,12 +446,17 @@ int gx_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int heads, 
  * thread of a workgroup takes a share of both sums, where golem's order
  * leaves them to one lane per head and one per head element.  Same
  * arguments, caches and outputs as the serial forms; the caches come out bit
- * for bit the same.  A prompt (M > 4 tokens of one conversation, prefixes
- * of at most 1024) runs on the matrix cores instead: the scores and the
- * value sums are fp16 MFMA products (exact products, fp32 sums in the
- * matrix core's order), the maximum, exponentials, total and fp16
+ * for bit the same.  A decode step past 768 positions runs as four launches
+ * spread over the prefix, the same order and so the same bits; it needs the
+ * whole of gx_qwen_attention_workspace_bytes (with what the serial passes
+ * need alone, M * heads rows of scores and probabilities, they run instead).
+ * A prompt (M > 4 tokens of one conversation) runs on the matrix cores: the
+ * scores and the value sums are fp16 MFMA products (exact products, fp32 sums
+ * in the matrix core's order), the maximum, exponentials, total and fp16
  * probabilities as above; the head outputs stay within 1e-4 of RMS of
- * golem's.  Longer prompts and batches with slots take the serial kernels. */
+ * golem's.  Past 1024 positions it sweeps the prefix three times instead of
+ * keeping the scores, to about 76,000 positions; longer prompts take the
+ * serial kernels. */
 int gx_qwen_attention_parallel(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int head_dim,
                                int max_pos, const int32_t *positions, const uint16_t *kcache,
                                const uint16_t *vcache, int context, int8_t *q, float *scales, int32_t *qsum,
