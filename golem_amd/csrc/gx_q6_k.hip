@@ -9,6 +9,8 @@
 // the weights, the role of dotQ6_Kx2 (nn/dot_q6_k_x2_amd64.s:64-154), and
 // give each column exactly its one-column result.
 //
+// One column (and inputs the second kernel does not take) runs on the vector
+// ALU, two to sixteen at a time on the matrix cores (below).
 // Decomposition as the Q4_0 kernel: a workgroup owns one 64-row tile, each
 // wavefront whole superblocks, a lane one row.  The activation of a
 // superblock is uniform across the wavefront and is read into SGPRs with
@@ -94,6 +96,199 @@ int launch_nc(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *ksc
     return check_launch("q6_k_matvec");
 }
 
+// ---- 2 to 16 columns on the matrix cores ------------------------------------
+//
+// v_mfma_i32_16x16x64_i8 takes 64 inputs of 16 rows against 16 columns, a
+// lane the 16 inputs of one of the row's four scale groups: the group's scale
+// is that lane's own, so it goes into the weights, (q - 32) * scale, 14 bits
+// and a sign, as 64 * h + l with h in [-64, 63] and l in [0, 63], two int8
+// operands.  A superblock's integer sum - 32*shift is then 64 * (the h
+// products) + (the l products), exactly, for every column at once; the rest
+// is the one-column kernel's arithmetic in its order: (float(isum) * d) *
+// kscale, added superblock by superblock, in the lane that holds the output.
+//
+// A workgroup owns 128 rows (two R64 tiles), a wavefront 16 of them and all
+// their superblocks, the next one's loads in flight under this one's
+// arithmetic.  A lane loads its row's chunk of its own group, so a load's 64
+// lanes cover four 256-byte runs.  The columns' inputs sit in LDS, rows K +
+// 16 bytes apart (no bank conflicts), with their scales and the rows' d.
+//
+// What bounds it: HBM (the bytes take 47 us at 151936 x 2560), beside the
+// widening (240 vector instructions per 16 rows and superblock).  2 / 4 / 6 /
+// 8 / 16 columns there: 60 / 61 / 61 / 62 / 67 us, where the vector kernel
+// above, its columns in turn, takes 61 / 72 / 132 / 115 / 225 (102 registers,
+// so one workgroup a CU, and scalar loads of the activation a column).  Four
+// wavefronts a workgroup: 60 / 62 / 79 us at 2 / 6 / 16; sixteen 67 / 69 / 75;
+// two superblocks ahead 63 / 65 / 71.
+constexpr int kColsWaves = 8, kColsRows = 16 * kColsWaves, kColsMax = 16;
+
+typedef short v2s __attribute__((ext_vector_type(2)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// Four 6-bit weights q (one a byte) times the scale, (q - 32) * scale = 256 h +
+// l: m = q * scale + (128 - 32 * scale) is 256 h + l + 128, so h is m's high
+// byte and l its low one with the top bit flipped.
+__device__ __forceinline__ void q6_scaled(uint32_t q, uint32_t sc2, uint32_t add2, int &h, int &l) {
+    const uint32_t e = __builtin_amdgcn_perm(0u, q, 0x0c020c00u), o = __builtin_amdgcn_perm(0u, q, 0x0c030c01u);
+    uint32_t me, mo;
+    asm("v_pk_mad_i16 %0, %1, %2, %3" : "=v"(me) : "v"(e), "v"(sc2), "v"(add2));
+    asm("v_pk_mad_i16 %0, %1, %2, %3" : "=v"(mo) : "v"(o), "v"(sc2), "v"(add2));
+    h = (int)__builtin_amdgcn_perm(mo, me, 0x07030501u);
+    l = (int)(__builtin_amdgcn_perm(mo, me, 0x06020400u) ^ 0x80808080u);
+}
+
+__host__ __device__ inline size_t q6_cols_lds(int M, int K, int B, int DC) {
+    return (size_t)M * (K + 16) + (size_t)M * B * 4 + (size_t)DC * 8 * kColsRows * 2;
+}
+
+template <bool DOTS>
+__global__ __launch_bounds__(64 * kColsWaves, 4) void q6_k_mfma_cols_kernel(
+    const uint8_t *__restrict__ W, size_t plane0_bytes, int B, int DC, const int8_t *__restrict__ q,
+    const float *__restrict__ kscales, int K, int M, int tiles, int tile0, int row_start, int row_end,
+    const float *__restrict__ bias, float *__restrict__ y, int ldy, int32_t *__restrict__ dots) {
+    extern __shared__ __align__(16) uint8_t lds[];  // inputs [M][K + 16], kscales [M][B], d [DC * 8][128]
+    float *ks = (float *)(lds + (size_t)M * (K + 16));
+    uint16_t *dl = (uint16_t *)(ks + M * B);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, g = lane >> 4;
+    const int T0 = tile0 + kColsRows / kTileRows * blockIdx.x, tile = min(T0 + (wave >> 2), tiles - 1);
+    const uint8_t *base = W + (size_t)tile * B * kQ6Chunks * kTileRows * kChunk;
+    const uint32_t row_off = (uint32_t)(16 * (wave & 3) + li) * kChunk;
+    uint32_t o_ql[2], o_qh[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; hh++) {
+        o_ql[hh] = (uint32_t)(4 * hh + g) * kTileRows * kChunk + row_off;
+        o_qh[hh] = (uint32_t)(8 + 2 * hh + (g & 1)) * kTileRows * kChunk + row_off;
+    }
+    const uint32_t o_sc = 12u * kTileRows * kChunk + row_off;
+    struct Super {
+        uint4 ql[2], qh[2], sc;
+    };
+    auto load = [&](Super &w, int s) __attribute__((always_inline)) {
+        const uint8_t *p = base + (size_t)s * kQ6Chunks * kTileRows * kChunk;
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            w.ql[hh] = load_stream(p + o_ql[hh]);
+            w.qh[hh] = load_stream(p + o_qh[hh]);
+        }
+        w.sc = load_stream(p + o_sc);
+    };
+    Super wa, wb;
+    load(wa, 0);
+
+    // the columns and scales into LDS
+    const int pieces = M * (K / 16);
+    for (int i = tid; i < pieces; i += 64 * kColsWaves) {
+        const int c = i / (K / 16), p = i - c * (K / 16);
+        *(v4u_stream *)(lds + (size_t)c * (K + 16) + 16 * p) = *(const v4u_stream *)(q + (size_t)c * K + 16 * p);
+    }
+    for (int i = tid; i < M * B; i += 64 * kColsWaves)
+        ks[i] = DOTS ? 0.0f : kscales[i];
+    for (int i = tid; i < kColsRows * DC; i += 64 * kColsWaves) {
+        const int r = i & (kColsRows - 1), c = i / kColsRows;
+        const v4u_stream v = *(const v4u_stream *)(W + plane0_bytes +
+                                                   (((size_t)min(T0 + (r >> 6), tiles - 1) * DC + c) * kTileRows + (r & 63)) *
+                                                       kChunk);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            dl[(8 * c + j) * kColsRows + r] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+    }
+    __syncthreads();
+
+    const int col = min(li, M - 1);  // a lane past the columns repeats the last: never stored
+    const uint8_t *act = lds + (size_t)col * (K + 16) + 16 * g;
+    const uint32_t sl = g < 2 ? 4 : 2, sh = g < 2 ? 0 : 2;
+    float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int row0 = T0 * kTileRows + 16 * wave + 4 * g;  // this lane's four outputs
+    auto step = [&](const Super &w, int s) __attribute__((always_inline)) {
+        const uint32_t scw[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
+        v4i Dh = {0, 0, 0, 0}, Dl = {0, 0, 0, 0};
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            const uint32_t L[4] = {w.ql[hh].x, w.ql[hh].y, w.ql[hh].z, w.ql[hh].w};
+            const uint32_t H[4] = {w.qh[hh].x, w.qh[hh].y, w.qh[hh].z, w.qh[hh].w};
+#pragma unroll
+            for (int hi = 0; hi < 2; hi++) {  // groups 8 hh + 4 hi + g: the low nibbles, then the high ones
+                const v4i bv = *(const v4i *)(act + (size_t)s * kSuper + 128 * hh + 64 * hi);
+                const int sc = (int)(scw[2 * hh + hi] << (24 - 8 * g)) >> 24;
+                const uint32_t sc2 = __builtin_amdgcn_perm(0u, (uint32_t)sc, 0x01000100u);
+                const v2s a2 = {(short)(128 - 32 * sc), (short)(128 - 32 * sc)};
+                const uint32_t add2 = __builtin_bit_cast(uint32_t, a2);
+                v4i h, l;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const uint32_t q6 = hi ? ((L[k] >> 4) & 0x0F0F0F0Fu) | ((H[k] >> sh) & 0x30303030u)
+                                           : (L[k] & 0x0F0F0F0Fu) | ((H[k] << sl) & 0x30303030u);
+                    int hk, lk;
+                    q6_scaled(q6, sc2, add2, hk, lk);
+                    h[k] = hk;
+                    l[k] = lk;
+                }
+                Dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(h, bv, Dh, 0, 0, 0);
+                Dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(l, bv, Dl, 0, 0, 0);
+            }
+        }
+        const uint2 dw = *(const uint2 *)(dl + s * kColsRows + 16 * wave + 4 * g);
+        const float kc = ks[col * B + s];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int32_t isum = (Dh[i] << 8) + Dl[i];
+            if constexpr (DOTS) {
+                const int r = row0 + i;
+                if (li < M && r >= row_start && r < row_end)
+                    dots[((size_t)li * (row_end - row_start) + (r - row_start)) * B + s] = isum;
+            } else {
+                const uint32_t dh = (i < 2 ? dw.x : dw.y) >> (16 * (i & 1));
+                const float t0 = (float)isum * half_bits_to_float(dh & 0xFFFFu);
+                const float t = t0 * kc;
+                total[i] = total[i] + t;
+            }
+        }
+    };
+    for (int s = 0; s < B; s += 2) {
+        load(wb, min(s + 1, B - 1));
+        step(wa, s);
+        if (s + 1 < B) {
+            load(wa, min(s + 2, B - 1));
+            step(wb, s + 1);
+        }
+    }
+    if (DOTS || li >= M)
+        return;
+    float *yr = y + (size_t)li * ldy;
+    if (bias) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            total[i] = total[i] + bias[min(row0 + i, row_end - 1)];
+    }
+    if (row0 >= row_start && row0 + 4 <= row_end && (ldy & 3) == 0 && ((uintptr_t)y & 15) == 0) {
+        *(float4 *)(yr + row0) = make_float4(total[0], total[1], total[2], total[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (row0 + i >= row_start && row0 + i < row_end)
+                yr[row0 + i] = total[i];
+    }
+}
+
+int launch_cols(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales, int M, int row_start,
+                int row_end, const float *bias, float *y, int ldy, int32_t *dots) {
+    const int tile0 = row_start / kTileRows;
+    const int grid = (row_end - tile0 * kTileRows + kColsRows - 1) / kColsRows;
+    const size_t lds = q6_cols_lds(M, w->cols, w->blocks, w->dchunks);
+#define GX_Q6_COLS(DD)                                                                                               \
+    q6_k_mfma_cols_kernel<DD><<<grid, 64 * kColsWaves, lds, ctx->stream>>>(                                          \
+        w->dev, w->plane0_bytes, w->blocks, w->dchunks, q, kscales, w->cols, M, w->tiles, tile0, row_start, row_end,  \
+        bias, y, ldy, dots)
+    if (dots)
+        GX_Q6_COLS(true);
+    else
+        GX_Q6_COLS(false);
+#undef GX_Q6_COLS
+    return check_launch("q6_k_mfma_cols");
+}
+
 }  // namespace
 
 int launch_q6_k_matvec(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales,
@@ -110,7 +305,14 @@ int launch_q6_k_matvec(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const f
         float *yc = y ? y + (size_t)c * ldy : nullptr;
         int32_t *dc = dots ? dots + (size_t)c * nrows * B : nullptr;
         int rc;
-        if (left >= 8) {
+        // Two columns or more on the matrix cores, sixteen a launch, where
+        // the inputs can be read 16 bytes at a time and their LDS leaves two
+        // workgroups a CU (sixteen columns of up to 4,608 inputs).
+        const int n = min(left, kColsMax);
+        if (left > 1 && ((uintptr_t)q & 15) == 0 && q6_cols_lds(n, K, B, w->dchunks) <= 80 * 1024) {
+            rc = launch_cols(ctx, w, qc, kc, n, row_start, row_end, bias, yc, ldy, dc);
+            c += n;
+        } else if (left >= 8) {
             rc = launch_nc<8>(ctx, w, qc, kc, bc, row_start, row_end, bias, yc, ldy, dc);
             c += 8;
         } else if (left >= 4) {

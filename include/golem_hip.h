@@ -172,7 +172,7 @@ int gx_matmul_q4_0_expert(gx_ctx *ctx, const gx_weight *w, int expert, const int
 /* y[m][r] = W[r] . x[m] (+ bias[r]) for a Q6_K matrix and a Q8_K batch:
  * MatVecQ6_K and matVecQ6_KRows (nn/dot_q6_k.go:64-103), which include the
  * two-column dotQ6_Kx2 (nn/dot_q6_k_amd64.go:14-20): one weight read serves
- * all M <= 8 columns.  Bit-identical to golem's dotQ6_KGo. */
+ * sixteen columns.  Bit-identical to golem's dotQ6_KGo. */
 int gx_matmul_q6_k(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales, const int16_t *bsums,
                    int M, int row_start, int row_end, const float *bias, float *y, int ldy);
 
