@@ -276,7 +276,7 @@ template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     const uint16_t *__restrict__ qh, int M, int heads, int kv_heads, const int32_t *__restrict__ positions,
     int limit, const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, int context, float scale,
-    int8_t *__restrict__ q, float *__restrict__ scales, int32_t *__restrict__ qsum) {
+    int8_t *__restrict__ q, float *__restrict__ scales, int32_t *__restrict__ qsum, float *__restrict__ heads_f) {
     constexpr int KS = HD / 16, DB = HD / 32;
     extern __shared__ __align__(16) float sl[];  // block sums [blocks][32]; at the end the value sums and the output tile
     __shared__ float mw[NW][kPlTok];
@@ -523,8 +523,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
         const uint32_t packed = q8_0_quad(v, &stored, &sm);
         if (t0 + tk < M) {
             const int col = h * HD + 4 * c4;
-            *(uint32_t *)(q + (size_t)(t0 + tk) * width + col) = packed;
-            if ((c4 & 7) == 0) {
+            if (heads_f)
+                *(float4 *)(heads_f + (size_t)(t0 + tk) * width + col) = o;
+            if (q) {
+                *(uint32_t *)(q + (size_t)(t0 + tk) * width + col) = packed;
+                if ((c4 & 7) != 0)
+                    continue;
                 scales[(size_t)(t0 + tk) * (width >> 5) + (col >> 5)] = stored;
                 qsum[(size_t)(t0 + tk) * (width >> 5) + (col >> 5)] = sm;
             }
@@ -546,7 +550,7 @@ bool attn_prompt_long_fits(int hd, int limit) { return prompt_long_lds(hd, 8, li
 
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
-                            float scale, int8_t *q, float *scales, int32_t *qsum) {
+                            float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f) {
     const dim3 grid((unsigned)heads, (unsigned)((M + kPlTok - 1) / kPlTok));
     const bool wide = (size_t)grid.x * grid.y <= 2 * (size_t)ctx->cu_count;
     const int nw = wide ? 8 : 4;
@@ -554,7 +558,7 @@ int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, i
 #define GX_PL(HH, WW)                                                                                                \
     attn_prompt_long_kernel<HH, WW><<<grid, 64 * WW, lds, ctx->stream>>>(qh, M, heads, kv_heads, positions, limit,   \
                                                                          kcache, vcache, context, scale, q, scales,  \
-                                                                         qsum)
+                                                                         qsum, heads_f)
 #define GX_PL_W(HH)                                                                                                  \
     do {                                                                                                             \
         if (wide)                                                                                                    \

@@ -176,7 +176,7 @@ size_t qwen_attention_workspace_least(int M, int heads, int max_pos); // what a 
 bool attn_prompt_long_fits(int hd, int limit);
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
-                            float scale, int8_t *q, float *scales, int32_t *qsum);
+                            float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f);
 size_t attn_split_workspace(int M, int heads, int S);
 int launch_attn_split(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
                       const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,

@@ -2211,13 +2211,19 @@ int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int
                                  q, scales, qsum, sc, (float *)prob,
                                  (float *)(workspace + qwen_attention_workspace_least(M, heads, max_pos)), slots,
                                  nslots);
-    // A prompt of one conversation in the parallel order: the matrix cores.
+    // A prompt of one conversation in the parallel order: the matrix cores,
+    // the scores in LDS while two workgroups a CU hold them (576 positions)
+    // or the tiles are few, in three sweeps past that.  32 heads of 128 (us,
+    // LDS / sweeps): 512 tokens 26 / 39, 300 after 500 54 / 53, 64 after 900
+    // 39 / 34, 8 after 900 25 / 33, 1000 tokens 135 / 78.
+    const bool sweeps = !slots && M > 4 && attn_prompt_long_fits(hd, limit) &&
+                        (limit > kPmMax || (limit > 576 && (size_t)((M + kPmTok - 1) / kPmTok) * heads > 32));
+    if (parallel && sweeps)
+        return launch_attn_prompt_long(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context,
+                                       scale, q, scales, qsum, heads_f);
     if (parallel && !slots && limit <= kPmMax)
         return launch_prompt_mfma(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context, scale,
                                   q, scales, qsum, heads_f);
-    if (parallel && !slots && M > 4 && attn_prompt_long_fits(hd, limit))
-        return launch_attn_prompt_long(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context,
-                                       scale, q, scales, qsum);
     if ((M <= 4 || slots) && limit <= kDecodeMax) {
 // One query head per workgroup when that fills at most two workgroups per CU
 // (128 workgroups for config 3's decode rather than 32): the scores,
