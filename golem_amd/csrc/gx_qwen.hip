@@ -95,12 +95,25 @@ __global__ __launch_bounds__(kQNormThreads) void qwen_norm_quant_kernel(float *_
     }
 }
 
-// RMSNormPlain of one head of hd floats held two per lane (lane owns i and
-// i + 64), the float64 sum taken left to right by lane 0 from LDS.
+// RMSNormPlain's scale of one head of hd floats (a multiple of 8), the
+// float64 sum taken left to right by one lane from LDS, sixteen values read
+// ahead of the sum.
 __device__ __forceinline__ float head_norm_scale(const float *h, int hd, float eps) {
     double s = 0.0;
-    for (int i = 0; i < hd; i++) {
-        const float v = h[i];
+    int i0 = 0;
+    for (; i0 + 16 <= hd; i0 += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            v[i] = h[i0 + i];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const float sq = v[i] * v[i];
+            s += (double)sq;
+        }
+    }
+    for (; i0 < hd; i0++) {
+        const float v = h[i0];
         const float sq = v * v;
         s += (double)sq;
     }
@@ -131,7 +144,6 @@ __global__ __launch_bounds__(64) void qwen_qk_rope_kernel(const float *__restric
                                                           uint16_t *__restrict__ vcache, int context,
                                                           const int32_t *__restrict__ slots, int nslots) {
     __shared__ float h[kHeadMax];
-    __shared__ float sc_sh;
     const int lane = threadIdx.x, t = blockIdx.x, u = blockIdx.y;
     const int pos = positions[t];
     // A position past the cache, or a slot that names no conversation, has
@@ -153,21 +165,54 @@ __global__ __launch_bounds__(64) void qwen_qk_rope_kernel(const float *__restric
     const bool is_q = u < heads;
     const int col = is_q ? u * hd : heads * hd + (u - heads) * hd;
     const float *src = qkv + (size_t)t * ldqkv + col;
-    for (int i = lane; i < hd; i += 64)
-        h[i] = src[i];
-    __syncthreads();
-    if (lane == 0)
-        sc_sh = head_norm_scale(h, hd, eps);
-    __syncthreads();
-    const float sc = sc_sh;
     const float *gain = is_q ? q_norm : k_norm;
+    // Every load goes out before the norm's serial sum: the lane's pairs
+    // (i, i + half) for i = lane and lane + 64, their gains and rotations,
+    // and a key-value head's values.  (Waiting for the sum before asking for
+    // the rest, and for each value of the sum, took 5.6 us at one token of 40
+    // heads of 128, this 3.9.)
+    constexpr int kPairs = kHeadMax / 2 / 64;
+    float x0[kPairs], x1[kPairs], g0[kPairs], g1[kPairs], cs[kPairs], sn[kPairs], vv[2 * kPairs];
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+        const int i = min(lane + 64 * k, half - 1);
+        x0[k] = src[i];
+        x1[k] = src[i + half];
+    }
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+        const int i = min(lane + 64 * k, half - 1);
+        g0[k] = gain[i];
+        g1[k] = gain[i + half];
+        cs[k] = rope_cos[(size_t)pos * half + i];
+        sn[k] = rope_sin[(size_t)pos * half + i];
+    }
+    if (!is_q) {
+        const float *vsrc = qkv + (size_t)t * ldqkv + (heads + kv_heads) * hd + (u - heads) * hd;
+#pragma unroll
+        for (int k = 0; k < 2 * kPairs; k++)
+            vv[k] = vsrc[min(lane + 64 * k, hd - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+        const int i = lane + 64 * k;
+        if (i < half) {
+            h[i] = x0[k];
+            h[i + half] = x1[k];
+        }
+    }
+    lds_barrier();
+    // every lane takes the same sum (broadcast reads)
+    const float sc = head_norm_scale(h, hd, eps);
     // normed, then rotated in pairs (i, i + half): RoPETable.Apply, nn/rope.go:62-73
-    for (int i = lane; i < half; i += 64) {
-        const float re0 = h[i], im0 = h[i + half];
-        const float re = (re0 * sc) * gain[i], im = (im0 * sc) * gain[i + half];
-        const float c = rope_cos[(size_t)pos * half + i], s = rope_sin[(size_t)pos * half + i];
-        const float a = re * c - im * s;
-        const float b = re * s + im * c;
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+        const int i = lane + 64 * k;
+        if (i >= half)
+            continue;
+        const float re = (x0[k] * sc) * g0[k], im = (x1[k] * sc) * g1[k];
+        const float a = re * cs[k] - im * sn[k];
+        const float b = re * sn[k] + im * cs[k];
         if (is_q) {
             qh[(size_t)t * heads * hd + u * hd + i] = (uint16_t)float_to_half_bits(a);
             qh[(size_t)t * heads * hd + u * hd + i + half] = (uint16_t)float_to_half_bits(b);
@@ -179,10 +224,13 @@ __global__ __launch_bounds__(64) void qwen_qk_rope_kernel(const float *__restric
         }
     }
     if (!is_q) {
-        const float *vsrc = qkv + (size_t)t * ldqkv + (heads + kv_heads) * hd + (u - heads) * hd;
         uint16_t *vt = vcache + (size_t)(u - heads) * hd * context + pos;
-        for (int i = lane; i < hd; i += 64)
-            vt[(size_t)i * context] = (uint16_t)float_to_half_bits(vsrc[i]);
+#pragma unroll
+        for (int k = 0; k < 2 * kPairs; k++) {
+            const int i = lane + 64 * k;
+            if (i < hd)
+                vt[(size_t)i * context] = (uint16_t)float_to_half_bits(vv[k]);
+        }
     }
 }
 
@@ -2147,6 +2195,8 @@ int launch_qwen_qk_rope(gx_ctx *ctx, const float *qkv, int ldqkv, int M, int hea
                         int context, const int32_t *slots, int nslots) {
     GX_CHECK(hd <= kHeadMax && hd % 8 == 0, "gx: head width %d unsupported (a multiple of 8, at most %d)", hd,
              kHeadMax);
+    if (hd <= 0)
+        return GX_OK;  // heads of no values: nothing to store
     // A batch (and a head width the tiled kernel is built for, operands it
     // can read 16 bytes at a time): 64 tokens of a head a workgroup.
     const bool aligned =
