@@ -28,35 +28,36 @@
 namespace gx {
 namespace {
 
-constexpr int kQNormThreads = 1024;
+constexpr int kQNormThreads = 1024;  // a row's threads while every CU has at most one row
 
 // One position per workgroup: x (and add) [M][ld], gain [K].  out, when given,
 // receives the normed floats [M][ldo]; q/scales/qsum receive its Q8_0 form.
 // RMSNormPlain's float64 sum is the tree of gx_device.hpp (512 partials,
 // partial t = elements t, t+512, ... in order, halved pairwise): threads
 // 0..511 stage x (+ add) and their partials (norm_stage) while threads
-// 512..1023 stage the gains, wavefront 0 takes the tree (norm_tree_wave) --
-// two barriers -- and the Q8_0 goes four values a lane, a block per eight
-// lanes (q8_0_quad).  (Against a five-barrier tree and one value a lane:
-// 6.3 -> 4.9 us at 8 positions of 2560.)
-__global__ __launch_bounds__(kQNormThreads) void qwen_norm_quant_kernel(float *__restrict__ x, int ldx,
-                                                                        const float *__restrict__ add, int lda,
-                                                                        const float *__restrict__ gain, int K,
-                                                                        float eps, float *__restrict__ out, int ldo,
-                                                                        int8_t *__restrict__ q,
-                                                                        float *__restrict__ scales,
-                                                                        int32_t *__restrict__ qsum) {
-    extern __shared__ __align__(16) float xs[];  // K floats, then the K gains
+// 512..1023, where there are as many, stage the gains (else they are read in
+// place), wavefront 0 takes the tree (norm_tree_wave) -- two barriers -- and
+// the Q8_0 goes four values a lane, a block per eight lanes (q8_0_quad).
+// (Against a five-barrier tree and one value a lane: 6.3 -> 4.9 us at 8
+// positions of 2560.)
+template <int NT>
+__global__ __launch_bounds__(NT) void qwen_norm_quant_kernel(float *__restrict__ x, int ldx,
+                                                             const float *__restrict__ add, int lda,
+                                                             const float *__restrict__ gain, int K, float eps,
+                                                             float *__restrict__ out, int ldo,
+                                                             int8_t *__restrict__ q, float *__restrict__ scales,
+                                                             int32_t *__restrict__ qsum) {
+    extern __shared__ __align__(16) float xs[];  // K floats, then (NT 1024) the K gains
     float *gl = xs + K;
     __shared__ double red[512];
     __shared__ float scale_sh;
     const int tid = threadIdx.x, t = blockIdx.x;
     float *xr = x + (size_t)t * ldx;
     const float *ar = add ? add + (size_t)t * lda : nullptr;
-    if (tid < 512) {
+    if (NT < 1024 || tid < 512) {
         norm_stage(xr, ar, K, xs, ar ? xr : nullptr, red);  // x + add written back as the residual
     } else {
-        for (int i = tid - 512; i < K; i += kQNormThreads - 512)
+        for (int i = tid - 512; i < K; i += NT - 512)
             gl[i] = gain[i];
     }
     __syncthreads();
@@ -68,9 +69,10 @@ __global__ __launch_bounds__(kQNormThreads) void qwen_norm_quant_kernel(float *_
     __syncthreads();
     const float sc = scale_sh;
     const int B = K >> 5;
-    for (int i4 = tid; i4 < K / 4; i4 += kQNormThreads) {  // K % 32 == 0: whole eight-lane groups in or out
+    for (int i4 = tid; i4 < K / 4; i4 += NT) {  // K % 32 == 0: whole eight-lane groups in or out
         const float4 xv = ((const float4 *)xs)[i4];
-        const float4 gv = ((const float4 *)gl)[i4];
+        const float4 gv = NT < 1024 ? make_float4(gain[4 * i4], gain[4 * i4 + 1], gain[4 * i4 + 2], gain[4 * i4 + 3])
+                                    : ((const float4 *)gl)[i4];
         float nv[4];
         nv[0] = (xv.x * sc) * gv.x;
         nv[1] = (xv.y * sc) * gv.y;
@@ -2184,8 +2186,20 @@ int launch_qwen_norm_quant(gx_ctx *ctx, float *x, int ldx, const float *add, int
                            float eps, float *out, int ldo, int8_t *q, float *scales, int32_t *qsum) {
     const size_t lds = 2 * sizeof(float) * (size_t)K;
     GX_CHECK(lds <= 160 * 1024, "gx: a norm over %d values does not fit the LDS", K);
-    qwen_norm_quant_kernel<<<M, kQNormThreads, lds, ctx->stream>>>(x, ldx, add, lda, gain, K, eps, out, ldo, q,
-                                                                   scales, qsum);
+    // A row is a chain of latencies, so rows past one a CU are worth more side
+    // by side than each spread wide (us at 1024 / 512 / 256 threads, 2560
+    // wide: 200 rows 4.5/4.7/4.8, 500 rows 5.6/4.5/5.0, 600 7.0/4.9/5.3, 800
+    // 9.0/6.5/5.9, 1500 13.6/8.6/7.7, 4096 33.6/19.2/15.8; 128 threads are
+    // slower at every count).
+    if (M > 3 * ctx->cu_count)
+        qwen_norm_quant_kernel<256><<<M, 256, lds / 2, ctx->stream>>>(x, ldx, add, lda, gain, K, eps, out, ldo, q,
+                                                                      scales, qsum);
+    else if (M > ctx->cu_count)
+        qwen_norm_quant_kernel<512><<<M, 512, lds / 2, ctx->stream>>>(x, ldx, add, lda, gain, K, eps, out, ldo, q,
+                                                                      scales, qsum);
+    else
+        qwen_norm_quant_kernel<kQNormThreads><<<M, kQNormThreads, lds, ctx->stream>>>(
+            x, ldx, add, lda, gain, K, eps, out, ldo, q, scales, qsum);
     return check_launch("qwen_norm_quant");
 }
 
