@@ -271,6 +271,7 @@ typedef float pl_v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t pl_v2u __attribute__((ext_vector_type(2)));
 
 constexpr int kPlTok = 32;
+constexpr int kPlOne = 1024;  // positions the LDS form takes
 
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
@@ -286,7 +287,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     // read the same keys), the longest prefixes first
     const int kvh = blockIdx.x % kv_heads, h = kvh * (heads / kv_heads) + blockIdx.x / kv_heads;
     const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kPlTok, t = t0 + li;
-    const int n = t < M ? max(min(positions[t] + 1, limit), 0) : 0;  // this lane's token's positions
+    // this lane's token's positions (a negative position: as the LDS form to
+    // 1024 positions, one; as the serial passes past them, none)
+    const int n = t < M ? max(min(positions[t] + 1, limit), limit <= kPlOne ? 1 : 0) : 0;
     int nmax = n, nmin = t < M ? n : limit;
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) {
@@ -426,20 +429,10 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     for (int db = 0; db < DB; db++)
         acc[db] = pl_v16f{};
     const char *vb = (const char *)(vcache + (size_t)kvh * HD * context);  // 32-bit offsets, as the keys'
-    sweep([&](int p0, const float *s, int) __attribute__((always_inline)) {
-        pl_v2u v[DB][2][2];  // [element block][k-step][positions 4 g .., 8 + 4 g ..]
-#pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int st = 0; st < 2; st++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-                    v[db][st][u] = *(const pl_v2u *)(vb + ((uint32_t)((32 * db + li) * context +
-                                                                      min(p0 + 16 * st + 8 * u + 4 * g, context - 4)) *
-                                                           2u));
+    // a tile's probabilities, fp16 pairs
+    auto probs = [&](int p0, const float *s, uint32_t *ph) __attribute__((always_inline)) {
         float e16[16];
         exps(p0, s, e16);
-        uint32_t ph[8];  // probabilities, fp16 pairs
 #pragma unroll
         for (int e = 0; e < 16; e += 2) {
             ph[e >> 1] = float_to_half_bits(__fdiv_rn(e16[e], total)) |
@@ -452,6 +445,50 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
             for (int e = 0; e < 16; e += 2)
                 ph[e >> 1] &= (in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u);
         }
+    };
+    auto vload = [&](int p0, int db, int st, int u) __attribute__((always_inline)) {
+        return *(const pl_v2u *)(vb + ((uint32_t)((32 * db + li) * context +
+                                                  min(p0 + 16 * st + 8 * u + 4 * g, context - 4)) *
+                                       2u));
+    };
+    // A later token's infinite or NaN value must not reach an earlier one as
+    // 0 * inf: the wavefront's tiles from the first with such a value past
+    // some token's own positions wait.  (Looked for ahead of the sweep: in it,
+    // where the values are at hand, it spilled, 172 -> 186 us.)
+    int late = nmax;
+    int b0 = wave;
+    while (b0 < nb && (b0 + 1) * kBlock <= nmin)
+        b0 += NW;
+#pragma unroll 1
+    for (int p0 = b0 * kBlock; p0 < late; p0 += (p0 & 32) ? NW * kBlock - 32 : 32) {
+        const int own = left(p0, nmax);
+        uint32_t any = 0;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int w = 0; w < 8; w++) {
+                const int e = 2 * w;
+                const uint32_t keep = (in(own, e) ? 0x7FFFu : 0u) | (in(own, e + 1) ? 0x7FFF0000u : 0u);
+                // an exponent of all ones carries into the half's sign place
+                any |= ((vload(p0, db, w >> 2, (w >> 1) & 1)[w & 1] & keep) + 0x04000400u) & 0x80008000u;
+            }
+        if (p0 + 32 > nmin && __ballot(any != 0) != 0)
+            late = p0;
+    }
+    late = __builtin_amdgcn_readfirstlane(late);
+    sweep([&](int p0, const float *s, int) __attribute__((always_inline)) {
+        if (p0 >= late)
+            return;
+        pl_v2u v[DB][2][2];  // [element block][k-step][positions 4 g .., 8 + 4 g ..]
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int st = 0; st < 2; st++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    v[db][st][u] = vload(p0, db, st, u);
+        uint32_t ph[8];
+        probs(p0, s, ph);
         if (p0 + 32 > nmax) {  // values past the tile's last position may be unwritten: zeros
             const int own = left(p0, nmax);
 #pragma unroll
@@ -478,6 +515,48 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
             }
         }
     });
+
+    // the tiles that waited, a token at a time with the values past it zeroed
+#pragma unroll 1
+    for (int p0 = late; p0 < nmax; p0 += (p0 & 32) ? NW * kBlock - 32 : 32) {
+        uint32_t ph[8];
+        {
+            pl_v8h k[KS];
+            float s[16];
+            kload(p0, k);
+            score(k, s);
+            probs(p0, s, ph);
+        }
+#pragma unroll 1
+        for (int tt = 0; tt < kPlTok; tt++) {
+            const int own = left(p0, __builtin_amdgcn_readlane(n, tt));
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                pl_v16f one = acc[db];
+#pragma unroll
+                for (int st = 0; st < 2; st++) {
+                    uint32_t vm[4];
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        const pl_v2u x = vload(p0, db, st, u);
+#pragma unroll
+                        for (int c = 0; c < 2; c++) {
+                            const int e = 8 * st + 4 * u + 2 * c;
+                            vm[2 * u + c] =
+                                x[c] & ((in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u));
+                        }
+                    }
+                    const uint4 pb = make_uint4(ph[4 * st], ph[4 * st + 1], ph[4 * st + 2], ph[4 * st + 3]);
+                    const uint4 va = make_uint4(vm[0], vm[1], vm[2], vm[3]);
+                    one = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pl_v8h, va),
+                                                                 __builtin_bit_cast(pl_v8h, pb), one, 0, 0, 0);
+                }
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    acc[db][e] = li == tt ? one[e] : acc[db][e];
+            }
+        }
+    }
 
     // the wavefronts' sums: the upper half's added to the lower half's
     __syncthreads();  // the block sums are spent
@@ -544,10 +623,13 @@ size_t prompt_long_lds(int hd, int nw, int limit) {
 
 }  // namespace
 
+// The block sums have to fit the LDS, a key-value head's cache a 32-bit offset.
+bool attn_prompt_long_fits(int hd, int limit, int context) {
+    return prompt_long_lds(hd, 8, limit) <= 150 * 1024 && (uint64_t)hd * context * sizeof(uint16_t) <= 1u << 31;
+}
+
 // Wavefronts a workgroup: eight while the tiles would leave CUs without one,
 // four (two workgroups a CU) otherwise.
-bool attn_prompt_long_fits(int hd, int limit) { return prompt_long_lds(hd, 8, limit) <= 150 * 1024; }
-
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                             float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f) {

@@ -173,7 +173,7 @@ int launch_qwen_qk_rope(gx_ctx *ctx, const float *qkv, int ldqkv, int M, int hea
                         int context, const int32_t *slots, int nslots);
 size_t qwen_attention_workspace(int M, int heads, int max_pos);       // what the calls' callers allocate
 size_t qwen_attention_workspace_least(int M, int heads, int max_pos); // what a call cannot do without
-bool attn_prompt_long_fits(int hd, int limit);
+bool attn_prompt_long_fits(int hd, int limit, int context);
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                             float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f);

@@ -2280,7 +2280,7 @@ int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int
     // or the tiles are few, in three sweeps past that.  32 heads of 128 (us,
     // LDS / sweeps): 512 tokens 26 / 39, 300 after 500 54 / 53, 64 after 900
     // 39 / 34, 8 after 900 25 / 33, 1000 tokens 135 / 78.
-    const bool sweeps = !slots && M > 4 && attn_prompt_long_fits(hd, limit) &&
+    const bool sweeps = !slots && M > 4 && attn_prompt_long_fits(hd, limit, context) &&
                         (limit > kPmMax || (limit > 576 && (size_t)((M + kPmTok - 1) / kPmTok) * heads > 32));
     if (parallel && sweeps)
         return launch_attn_prompt_long(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context,

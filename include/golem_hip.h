@@ -454,9 +454,10 @@ int gx_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int heads, 
  * scores and the value sums are fp16 MFMA products (exact products, fp32 sums
  * in the matrix core's order), the maximum, exponentials, total and fp16
  * probabilities as above; the head outputs stay within 1e-4 of RMS of
- * golem's.  Past 1024 positions it sweeps the prefix three times instead of
- * keeping the scores, to about 76,000 positions; longer prompts take the
- * serial kernels. */
+ * golem's.  Past 1024 positions (past 576 where more than 32 workgroups
+ * share the work) it sweeps the prefix three times instead of keeping the
+ * scores, to about 76,000 positions; longer prompts take the serial
+ * kernels. */
 int gx_qwen_attention_parallel(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int head_dim,
                                int max_pos, const int32_t *positions, const uint16_t *kcache,
                                const uint16_t *vcache, int context, int8_t *q, float *scales, int32_t *qsum,

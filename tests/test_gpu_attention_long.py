@@ -138,3 +138,36 @@ def test_long_prompt_on_exact_scores(dev, orc, hd, heads, kv, M, start, context)
     assert np.abs(dq).max() <= 1 and np.count_nonzero(dq) <= max(3, dq.size // 1000)
     assert np.abs(sc[rows] / want.scales_rows() - 1).max() <= 2.0 ** -10
     np.testing.assert_array_equal(qs, q8.reshape(M, -1, 32).astype(np.int32).sum(2))
+
+
+@pytest.mark.parametrize("hd,start", [(128, 1100), (64, 600)])
+def test_long_prompt_keeps_later_infinities_out(dev, hd, start):
+    """An infinite and a NaN value of two tokens in mid-tile: the tokens before
+    them get the bits they get without them, the tokens after them everywhere
+    but in the blocks of the two elements."""
+    heads, kv, M = 16, 2, 70
+    n = start + M
+    context = (n + 7) // 8 * 8
+    g = synth.rng(hd)
+    k, v, kt, vt = _caches(g, 1, n, kv, hd, context, False)
+    qf = g.standard_normal((M, heads * hd)).astype(np.float16)
+    pos = np.arange(start, n, dtype=np.int32)
+    args = (heads, kv, hd, n - 1, context)
+    clean = _run(dev, "gx_qwen_attention_parallel", qf, pos, kt, vt, *args)
+    first, second = 13, 41  # tokens, of the first and the second tile
+    vt[0, 0, 5, start + first] = np.inf
+    vt[0, 1, hd - 1, start + second] = NAN
+    wild = _run(dev, "gx_qwen_attention_parallel", qf, pos, kt, vt, *args)
+    blocks = np.arange(heads * hd // 32) * 32
+    own = (blocks % hd + 31 - hd + 1 == 0), (blocks % hd == 0)  # the last block of a head, the first
+    hit = np.zeros((M, blocks.size), bool)
+    hit[first:] |= (blocks // hd < heads // kv) & own[1]
+    hit[second:] |= (blocks // hd >= heads // kv) & own[0]
+    for a, b in zip(clean, wild):
+        a, b = (_bits(u).reshape(M, blocks.size, -1) if u.dtype == np.float32 else u.reshape(M, blocks.size, -1)
+                for u in (a, b))
+        np.testing.assert_array_equal(a[~hit], b[~hit])
+    # the infinity reaches its block's scale at every later token (a Q8_0
+    # block's peak passes a NaN by, so the other's says nothing)
+    block = hit[M - 1] & (blocks // hd < heads // kv)
+    assert np.isinf(wild[1][first:, block]).all()
