@@ -100,12 +100,13 @@ int launch_nc(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *ksc
 //
 // v_mfma_i32_16x16x64_i8 takes 64 inputs of 16 rows against 16 columns, a
 // lane the 16 inputs of one of the row's four scale groups: the group's scale
-// is that lane's own, so it goes into the weights, (q - 32) * scale, 14 bits
-// and a sign, as 64 * h + l with h in [-64, 63] and l in [0, 63], two int8
-// operands.  A superblock's integer sum - 32*shift is then 64 * (the h
-// products) + (the l products), exactly, for every column at once; the rest
-// is the one-column kernel's arithmetic in its order: (float(isum) * d) *
-// kscale, added superblock by superblock, in the lane that holds the output.
+// is that lane's own, so it goes into the weights, (q - 32) * scale, at most
+// 32 * 128 in magnitude, as 256 * h + l with h in [-16, 16] and l in [-128,
+// 127], two int8 operands.  A superblock's integer sum - 32*shift is then 256
+// * (the h products) + (the l products), exactly, for every column at once;
+// the rest is the one-column kernel's arithmetic in its order: (float(isum) *
+// d) * kscale, added superblock by superblock, in the lane that holds the
+// output.
 //
 // A workgroup owns 128 rows (two R64 tiles), a wavefront 16 of them and all
 // their superblocks, the next one's loads in flight under this one's
@@ -137,9 +138,24 @@ __device__ __forceinline__ void q6_scaled(uint32_t q, uint32_t sc2, uint32_t add
     l = (int)(__builtin_amdgcn_perm(mo, me, 0x06020400u) ^ 0x80808080u);
 }
 
-__host__ __device__ inline size_t q6_cols_lds(int M, int K, int B, int DC) {
-    return (size_t)M * (K + 16) + (size_t)M * B * 4 + (size_t)DC * 8 * kColsRows * 2;
+// The workgroup's LDS: the inputs [M][K + 16], the column scales [M][B] and
+// the rows' d [DC * 8][128], each part from a multiple of 16 bytes (d is read
+// eight bytes at a time, whatever M and B).
+__host__ __device__ constexpr size_t q6_cols_scales(int M, int K) { return (size_t)M * (K + 16); }
+__host__ __device__ constexpr size_t q6_cols_d(int M, int K, int B) {
+    return q6_cols_scales(M, K) + ((size_t)M * B * 4 + 15) / 16 * 16;
 }
+__host__ __device__ constexpr size_t q6_cols_lds(int M, int K, int B, int DC) {
+    return q6_cols_d(M, K, B) + (size_t)DC * 8 * kColsRows * 2;
+}
+constexpr bool q6_cols_aligned() {
+    for (int M = 1; M <= kColsMax; M++)
+        for (int B = 1; B <= 64; B++)
+            if (q6_cols_scales(M, 256 * B) % 16 != 0 || q6_cols_d(M, 256 * B, B) % 16 != 0)
+                return false;
+    return true;
+}
+static_assert(q6_cols_aligned(), "every part of the LDS can be read at its access width");
 
 template <bool DOTS>
 __global__ __launch_bounds__(64 * kColsWaves, 4) void q6_k_mfma_cols_kernel(
@@ -147,8 +163,8 @@ __global__ __launch_bounds__(64 * kColsWaves, 4) void q6_k_mfma_cols_kernel(
     const float *__restrict__ kscales, int K, int M, int tiles, int tile0, int row_start, int row_end,
     const float *__restrict__ bias, float *__restrict__ y, int ldy, int32_t *__restrict__ dots) {
     extern __shared__ __align__(16) uint8_t lds[];  // inputs [M][K + 16], kscales [M][B], d [DC * 8][128]
-    float *ks = (float *)(lds + (size_t)M * (K + 16));
-    uint16_t *dl = (uint16_t *)(ks + M * B);
+    float *ks = (float *)(lds + q6_cols_scales(M, K));
+    uint16_t *dl = (uint16_t *)(lds + q6_cols_d(M, K, B));
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g = lane >> 4;
     const int T0 = tile0 + kColsRows / kTileRows * blockIdx.x, tile = min(T0 + (wave >> 2), tiles - 1);

@@ -9,9 +9,11 @@ pytestmark = pytest.mark.gpu
 
 # rows, cols, M, first row, spare floats a row of y: tiles' edges, one
 # superblock, odd and past eight of them (a scale chunk), a second launch of
-# one and of two columns, inputs wider than the LDS
+# one and of two columns, inputs wider than the LDS, an odd number of column
+# scales (columns times superblocks: 3 to 135)
 CASES = [(64, 256, 2, 0, 0), (1000, 2560, 6, 0, 1), (129, 2816, 16, 3, 0), (257, 768, 17, 0, 0),
-         (200, 2304, 18, 65, 4), (128, 6144, 16, 0, 0), (130, 512, 9, 0, 2)]
+         (200, 2304, 18, 65, 4), (128, 6144, 16, 0, 0), (130, 512, 9, 0, 2), (64, 256, 3, 0, 0), (130, 2816, 11, 0, 0),
+         (200, 2304, 7, 0, 0), (257, 2304, 15, 3, 0), (65, 768, 5, 0, 1)]
 
 
 @pytest.mark.parametrize("rows,cols,M,start,spare", CASES)
