@@ -81,13 +81,15 @@ __global__ __launch_bounds__(1024) void q6_k_matvec_kernel(
     }
 }
 
+constexpr size_t kMatvecLds = 64 * 1024;
+
 template <int NC>
 int launch_nc(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales, const int16_t *bsums,
               int row_start, int row_end, const float *bias, float *y, int ldy, int32_t *dots) {
     const int B = w->blocks;
     const int waves = min(B, 16);
     const size_t lds = dots ? 0 : (size_t)B * NC * kTileRows * sizeof(float);
-    GX_CHECK(lds <= 64 * 1024, "gx: a %d-input Q6_K row is wider than this kernel's LDS", w->cols);
+    GX_CHECK(lds <= kMatvecLds, "gx: a %d-input Q6_K row is wider than this kernel's LDS", w->cols);
     const int tile0 = row_start / kTileRows;
     const int grid = (row_end + kTileRows - 1) / kTileRows - tile0;
     q6_k_matvec_kernel<NC><<<grid, 64 * waves, lds, ctx->stream>>>(w->dev, w->plane0_bytes, B, w->dchunks, q,
@@ -305,6 +307,43 @@ int launch_cols(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *k
     return check_launch("q6_k_mfma_cols");
 }
 
+// How many of `left` columns the matrix cores take in one launch, 0 for none:
+// as many as leave the LDS to two workgroups a CU (sixteen of up to 4,608
+// inputs, fourteen of 5,120), where the inputs can be read 16 bytes at a time.
+// A workgroup's superblocks are a serial chain (2.5 us and 1.15 more each,
+// however few the rows), where the vector kernel spreads them over its
+// wavefronts but reads the weights again for its next power of two of
+// columns.  So nine columns and more always go here; of the others those the
+// vector kernel takes in several reads (7 in three; 3, 5 and 6 in two) where a
+// row has few superblocks or the workgroups reach a small part of the CUs (7),
+// half of them (5, 6) or three quarters (3); and those it takes in one read
+// (2, 4, 8) from the counts at which its registers cost it more than the
+// chain.  us vector / matrix cores over weights not in the caches, rows x
+// inputs: two columns 4096 x 2560 6.6 / 14.7, 98304 x 2560 38.5 / 38.6, 151936
+// x 2560 59.7 / 58.2; three 8192 x 2560 12.7 / 15.0, 24576 x 2560 24.5 / 17.5,
+// 256 x 1024 7.3 / 7.1; four 16384 x 2560 10.8 / 16.0, 65536 x 2816 33.6 /
+// 29.1, 151936 x 1024 23.2 / 27.3; five 16384 x 2560 17.8 / 15.6; six 4096 x
+// 4096 17.3 / 21.9, 16384 x 4096 23.3 / 22.4; seven 512 x 5120 23.7 / 26.0,
+// 1024 x 4096 22.4 / 21.7; eight 16384 x 4096 17.9 / 22.7, 24576 x 4096 31.1 /
+// 23.3, 4096 x 1024 9.9 / 7.8.
+int cols_on_mfma(gx_ctx *ctx, const gx_weight *w, int left, bool aligned, int row_start, int row_end) {
+    const int cus = ctx->cu_count, few_supers = 4;
+    const int groups = (row_end - row_start / kTileRows * kTileRows + kColsRows - 1) / kColsRows;
+    int n = min(left, kColsMax);
+    while (n > 1 && q6_cols_lds(n, w->cols, w->blocks, w->dchunks) > 80 * 1024)
+        n--;
+    if (n < 2 || !aligned)
+        return 0;
+    const bool few = w->blocks <= few_supers;
+    const bool pays = n >= 9             ? true
+                    : n == 7             ? w->blocks <= 3 * few_supers || groups >= cus / 32
+                    : n == 2             ? !few && groups >= 4 * cus
+                    : n == 4             ? !few && groups >= 2 * cus
+                    : n == 3 || n == 8   ? few || groups >= 3 * cus / 4
+                                         : few || groups >= cus / 2;
+    return pays ? n : 0;
+}
+
 }  // namespace
 
 int launch_q6_k_matvec(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales,
@@ -312,6 +351,8 @@ int launch_q6_k_matvec(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const f
                        int ldy, int32_t *dots) {
     const int K = w->cols, B = w->blocks;
     const size_t nrows = (size_t)(row_end - row_start);
+    // the vector kernel's LDS holds nc columns' terms (it stores integers directly)
+    auto fits = [&](int nc) { return dots || (size_t)B * nc * kTileRows * sizeof(float) <= kMatvecLds; };
     int c = 0;
     while (c < M) {
         const int left = M - c;
@@ -321,20 +362,17 @@ int launch_q6_k_matvec(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const f
         float *yc = y ? y + (size_t)c * ldy : nullptr;
         int32_t *dc = dots ? dots + (size_t)c * nrows * B : nullptr;
         int rc;
-        // Two columns or more on the matrix cores, sixteen a launch, where
-        // the inputs can be read 16 bytes at a time and their LDS leaves two
-        // workgroups a CU (sixteen columns of up to 4,608 inputs).
-        const int n = min(left, kColsMax);
-        if (left > 1 && ((uintptr_t)q & 15) == 0 && q6_cols_lds(n, K, B, w->dchunks) <= 80 * 1024) {
+        const int n = cols_on_mfma(ctx, w, left, (uintptr_t)q % 16 == 0, row_start, row_end);
+        if (n) {
             rc = launch_cols(ctx, w, qc, kc, n, row_start, row_end, bias, yc, ldy, dc);
             c += n;
-        } else if (left >= 8) {
+        } else if (left >= 8 && fits(8)) {
             rc = launch_nc<8>(ctx, w, qc, kc, bc, row_start, row_end, bias, yc, ldy, dc);
             c += 8;
-        } else if (left >= 4) {
+        } else if (left >= 4 && fits(4)) {
             rc = launch_nc<4>(ctx, w, qc, kc, bc, row_start, row_end, bias, yc, ldy, dc);
             c += 4;
-        } else if (left >= 2) {
+        } else if (left >= 2 && fits(2)) {
             rc = launch_nc<2>(ctx, w, qc, kc, bc, row_start, row_end, bias, yc, ldy, dc);
             c += 2;
         } else {

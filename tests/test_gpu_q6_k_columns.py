@@ -1,5 +1,6 @@
-"""The Q6_K product's 2 to 16 columns on the matrix cores: each column bit for
-bit what the one-column kernel gives it, outputs and superblock integers."""
+"""The Q6_K product of several columns, on the matrix cores and in the vector
+kernel's wider forms: each column bit for bit what the one-column kernel gives
+it, outputs and superblock integers."""
 import numpy as np
 import pytest
 
@@ -7,13 +8,18 @@ from golem_amd import capi, synth
 
 pytestmark = pytest.mark.gpu
 
-# rows, cols, M, first row, spare floats a row of y: tiles' edges, one
-# superblock, odd and past eight of them (a scale chunk), a second launch of
-# one and of two columns, inputs wider than the LDS, an odd number of column
-# scales (columns times superblocks: 3 to 135)
-CASES = [(64, 256, 2, 0, 0), (1000, 2560, 6, 0, 1), (129, 2816, 16, 3, 0), (257, 768, 17, 0, 0),
-         (200, 2304, 18, 65, 4), (128, 6144, 16, 0, 0), (130, 512, 9, 0, 2), (64, 256, 3, 0, 0), (130, 2816, 11, 0, 0),
-         (200, 2304, 7, 0, 0), (257, 2304, 15, 3, 0), (65, 768, 5, 0, 1)]
+# rows, cols, M, first row, spare floats a row of y.  On the matrix cores:
+# tiles' edges, one superblock, odd and past eight of them (a scale chunk), a
+# second launch of one and of two columns, an odd number of column scales
+# (columns times superblocks: 3 to 135), inputs of which fourteen columns fit
+# the LDS, few columns of many rows.  On the vector kernel: 2, 3, 4, 6, 7 and 8
+# columns, eight and nine of a row that only its four fit
+CASES = [(64, 256, 3, 0, 0), (1000, 2560, 9, 0, 1), (129, 2816, 16, 3, 0), (257, 768, 17, 0, 0),
+         (200, 2304, 18, 65, 4), (130, 512, 9, 0, 2), (130, 2816, 11, 0, 0), (200, 2304, 7, 0, 0),
+         (257, 2304, 15, 3, 0), (65, 768, 5, 0, 1), (70, 5120, 16, 0, 0), (24600, 1280, 3, 5, 0),
+         (24600, 1280, 8, 0, 0), (64, 256, 2, 0, 0), (1000, 2560, 6, 0, 1), (130, 2816, 3, 0, 0),
+         (130, 2816, 4, 0, 0), (70, 2560, 8, 0, 0), (70, 5120, 7, 0, 0), (66, 8704, 8, 0, 0), (66, 8704, 9, 0, 0),
+         (128, 6144, 16, 0, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,M,start,spare", CASES)
