@@ -28,116 +28,138 @@ __device__ __forceinline__ float fma_mix_hi(uint32_t a, uint32_t b, float c) {
     return r;
 }
 
+constexpr int kOne = 1024;          // positions a prompt's LDS form takes (gx_qwen.hip)
+constexpr int kSplitTokens = 16;    // tokens the split form takes
+constexpr int kSplitWaves = 16384;  // wavefronts a launch of it (split_share)
 constexpr int kBlock = 64;  // positions a block of the softmax total
 constexpr int kRun = 32;    // positions a run of the value sums
 
 // ---- one position at a time (M <= 4, or one per conversation) ---------------
 //
-// Four launches, each spread over the prefix, so that the step's time does not
-// grow with it until the chip is full: the scores (a wavefront a head and 64
-// positions) with each block's maximum; the exponentials with each block's
-// sum; the probabilities and the runs' value chains; the runs in order with
-// the Q8_0.  The order of every sum is attn_par_kernel's, whatever the
-// extent.  What bounds it: the launches (about 2 us each) and their load
-// latencies; the bytes of 3,000 positions (12 MB) take 2 us.  The serial
-// passes it replaces took 104 us there (one lane's 3,000-step softmax total
-// 59, the value chains 38); these take 4.8 + 2.8 + 7.7 + 4.6.
+// Four launches, each spread over the prefix: the scores (a wavefront a head
+// and 64 positions) with each block's maximum; the exponentials with each
+// block's sum; the probabilities and the runs' value chains; the runs in order
+// with the Q8_0.  The order of every sum is attn_par_kernel's, whatever the
+// extent.  The grids' slowest dimension is the prefix, so that the workgroups
+// with positions come first and on different CUs: with the tokens slowest, the
+// empty ones between put every token's first block on the same few (sixteen
+// conversations at position 20, launched for 1,024: 24.7 us, now 15.0).
+// What bounds it: the launches (about 2 us each) and their load latencies;
+// then the bytes and two serial sums that every workgroup or lane repeats, a
+// prefix's blocks and its runs.  One position of 32 heads of 128 at 20 / 1,000
+// / 3,000 / 16,000 / 32,000: 14 / 15 / 20 / 43 / 80 us, where the serial
+// passes take 14 / 40 / 102 / 485 / 937.
 
-// grid (kv_heads, S / 64, tokens), 64 threads a query head of the group.
+// grid (kv_heads, tokens, blocks' share), 64 threads a query head of the group:
+// blocks blockIdx.z, blockIdx.z + share, ..
 template <int HD>
 __global__ __launch_bounds__(512) void attn_split_scores_kernel(
     const uint16_t *__restrict__ qh, int heads, int kv_heads, const int32_t *__restrict__ positions, int limit,
     const uint16_t *__restrict__ kcache, int context, float scale, int S, float *__restrict__ sc,
-    float *__restrict__ mx, const int32_t *__restrict__ slots, int nslots) {
+    float *__restrict__ mx, const int32_t *__restrict__ slots, int nslots, int share) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kvh = blockIdx.x, b = blockIdx.y, t = blockIdx.z;
+    const int kvh = blockIdx.x, t = blockIdx.y;
     const int h = kvh * (heads / kv_heads) + wave;
     const int n = min(positions[t] + 1, limit);
-    if (b * kBlock >= n)
-        return;
     if (slots)
         kcache += (size_t)min(max(slots[t], 0), nslots - 1) * kv_heads * HD * context;
-    const int p = b * kBlock + lane;
-    const v4u_stream *kr = (const v4u_stream *)(kcache + (size_t)kvh * HD * context) + min(p, n - 1);
-    v4u_stream k[HD / 8];
-#pragma unroll
-    for (int i = 0; i < HD / 8; i++)
-        k[i] = kr[(size_t)i * context];
     // the query is one address for the wavefront
     const v4u_stream *qv = (const v4u_stream *)(qh + ((size_t)t * heads + h) * HD);
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < HD / 8; i++) {
-        const v4u_stream qq = qv[i], kk = k[i];
-        s0 = fma_mix_lo(qq.x, kk.x, s0);
-        s1 = fma_mix_hi(qq.x, kk.x, s1);
-        s2 = fma_mix_lo(qq.y, kk.y, s2);
-        s3 = fma_mix_hi(qq.y, kk.y, s3);
-        s0 = fma_mix_lo(qq.z, kk.z, s0);
-        s1 = fma_mix_hi(qq.z, kk.z, s1);
-        s2 = fma_mix_lo(qq.w, kk.w, s2);
-        s3 = fma_mix_hi(qq.w, kk.w, s3);
-    }
-    const float v = scale * ((s0 + s1) + (s2 + s3));
     const size_t row = (size_t)t * heads + h;
-    if (p < n)
-        sc[row * S + p] = v;
-    const float m = wave_max(p < n ? v : -INFINITY);
-    if (lane == 0)
-        mx[row * (S / kBlock) + b] = m;
+    for (int b = blockIdx.z; b * kBlock < n; b += share) {
+        const int p = b * kBlock + lane;
+        const v4u_stream *kr = (const v4u_stream *)(kcache + (size_t)kvh * HD * context) + min(p, n - 1);
+        v4u_stream k[HD / 8];
+#pragma unroll
+        for (int i = 0; i < HD / 8; i++)
+            k[i] = kr[(size_t)i * context];
+        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < HD / 8; i++) {
+            const v4u_stream qq = qv[i], kk = k[i];
+            s0 = fma_mix_lo(qq.x, kk.x, s0);
+            s1 = fma_mix_hi(qq.x, kk.x, s1);
+            s2 = fma_mix_lo(qq.y, kk.y, s2);
+            s3 = fma_mix_hi(qq.y, kk.y, s3);
+            s0 = fma_mix_lo(qq.z, kk.z, s0);
+            s1 = fma_mix_hi(qq.z, kk.z, s1);
+            s2 = fma_mix_lo(qq.w, kk.w, s2);
+            s3 = fma_mix_hi(qq.w, kk.w, s3);
+        }
+        const float v = scale * ((s0 + s1) + (s2 + s3));
+        if (p < n)
+            sc[row * S + p] = v;
+        const float m = wave_max(p < n ? v : -INFINITY);
+        if (lane == 0)
+            mx[row * (S / kBlock) + b] = m;
+    }
 }
 
-// grid (S / 256, heads, tokens), a wavefront a block: exponentials in place.
-__global__ __launch_bounds__(256) void attn_split_exp_kernel(int heads, const int32_t *__restrict__ positions,
-                                                             int limit, int S, float *__restrict__ sc,
-                                                             const float *__restrict__ mx, float *__restrict__ bs) {
-    const int lane = threadIdx.x & 63, b = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int t = blockIdx.z;
-    const int n = min(positions[t] + 1, limit), nb = (n + kBlock - 1) / kBlock;
-    if (b >= nb)
+// grid (heads, tokens, blocks' share), four wavefronts, each with every fourth
+// of the workgroup's blocks: exponentials in place.
+__global__ __launch_bounds__(256) void attn_split_exp_kernel(int heads, int kv_heads,
+                                                             const int32_t *__restrict__ positions, int limit, int S,
+                                                             float *__restrict__ sc, const float *__restrict__ mx,
+                                                             float *__restrict__ bs, int share) {
+    const int lane = threadIdx.x & 63, b0 = blockIdx.z * 4 + (threadIdx.x >> 6);
+    const int t = blockIdx.y;
+    const int n = min(positions[t] + 1, limit), nb = n > 0 ? (n + kBlock - 1) / kBlock : 0;
+    if (b0 >= nb)
         return;
-    const size_t row = (size_t)t * heads + blockIdx.y;
-    const int p = b * kBlock + lane;
+    // key-value heads fastest: on the XCD that wrote the scores, where there are eight
+    const int h = (int)blockIdx.x % kv_heads * (heads / kv_heads) + (int)blockIdx.x / kv_heads;
+    const size_t row = (size_t)t * heads + h;
     float *s = sc + row * S;
-    const float v = s[min(p, n - 1)];
+    float v = s[min(b0 * kBlock + lane, n - 1)];
     const float *mr = mx + row * (S / kBlock);
     float m = -INFINITY;
     for (int i = lane; i < nb; i += 64)
         m = fmaxf(m, mr[i]);
     m = wave_max(m);
-    const float e = p < n ? exp_neg(v - m) : 0.0f;
-    s[p] = e;  // S is a whole number of blocks
-    const float sum = wave_pairwise_sum(e);
-    if (lane == 0)
-        bs[row * (S / kBlock) + b] = sum;
+    for (int b = b0;;) {
+        const int p = b * kBlock + lane;
+        const float e = p < n ? exp_neg(v - m) : 0.0f;
+        s[p] = e;  // S is a whole number of blocks
+        const float sum = wave_pairwise_sum(e);
+        if (lane == 0)
+            bs[row * (S / kBlock) + b] = sum;
+        b += 4 * share;
+        if (b >= nb)
+            break;
+        v = s[min(b * kBlock + lane, n - 1)];
+    }
 }
 
-// grid (kv_heads, S / (32 RW), tokens), RW * HD threads: run r of RW, element
-// d; the group's heads share the thread's 32 values.
+// grid (heads / G, tokens, the positions' share), RW * HD threads: run r of RW,
+// element d; G heads of a key-value head share the thread's 32 values.  (Eight
+// query heads a key-value head go four a workgroup: with a run's eight chains
+// in turn the step took 16.6 us at a prefix of 20, now 14.2.)
 template <int HD, int G>
 __global__ __launch_bounds__(256) void attn_split_values_kernel(
     int heads, int kv_heads, const int32_t *__restrict__ positions, int limit, const uint16_t *__restrict__ vcache,
     int context, int S, const float *__restrict__ sc, const float *__restrict__ bs, float *__restrict__ runs,
-    const int32_t *__restrict__ slots, int nslots) {
+    const int32_t *__restrict__ slots, int nslots, int share) {
     constexpr int RW = 256 / HD, NT = RW * HD, kPos = RW * kRun;
     __shared__ float bl[G][256];
     __shared__ float tot[G];
     __shared__ __align__(16) uint16_t ps[G][kPos];
     const int tid = threadIdx.x;
-    const int kvh = blockIdx.x, p0 = blockIdx.y * kPos, t = blockIdx.z;
+    const int h0 = blockIdx.x * G, kvh = h0 / (heads / kv_heads), t = blockIdx.y, step = share * kPos;
     const int n = min(positions[t] + 1, limit), nb = (n + kBlock - 1) / kBlock;
-    if (p0 >= n)
+    if ((int)blockIdx.z * kPos >= n)
         return;
     if (slots)
         vcache += (size_t)min(max(slots[t], 0), nslots - 1) * kv_heads * HD * context;
-    const size_t row0 = (size_t)t * heads + kvh * G;
+    const size_t row0 = (size_t)t * heads + h0;
     const int d = tid % HD, r = tid / HD;
-    const int pr = p0 + r * kRun;  // the thread's run
     const uint16_t *vrow = vcache + ((size_t)kvh * HD + d) * context;
     v4u_stream v[4];
+    auto vload = [&](int pr) __attribute__((always_inline)) {  // the run from position pr
 #pragma unroll
-    for (int u = 0; u < 4; u++)  // context is a multiple of 8; pieces past the prefix are read and not used
-        v[u] = *(const v4u_stream *)(vrow + min(pr + 8 * u, context - 8));
+        for (int u = 0; u < 4; u++)  // context is a multiple of 8; pieces past the prefix are read and not used
+            v[u] = *(const v4u_stream *)(vrow + min(pr + 8 * u, context - 8));
+    };
+    vload(blockIdx.z * kPos + r * kRun);
     // the heads' totals, blocks in order, 256 blocks at a time
     float total = 0.0f;  // thread g < G: head g's
     for (int c0 = 0; c0 < nb; c0 += 256) {
@@ -165,37 +187,42 @@ __global__ __launch_bounds__(256) void attn_split_values_kernel(
     }
     if (tid < G)
         tot[tid] = total;
-    __syncthreads();
-    for (int i = tid; i < G * kPos; i += NT) {
-        const int g = i / kPos, p = i - g * kPos;
-        ps[g][p] = p0 + p < n
-                       ? (uint16_t)float_to_half_bits(__fdiv_rn(sc[(row0 + g) * S + p0 + p], tot[g]))
-                       : (uint16_t)0;
-    }
-    __syncthreads();
-    const int live = min(kRun, n - pr);  // the run's positions
-    if (live <= 0)
-        return;
-    float acc[G];
-#pragma unroll
-    for (int g = 0; g < G; g++)
-        acc[g] = 0.0f;
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const uint32_t vw[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const v4u_stream pp = *(const v4u_stream *)(&ps[g][r * kRun + 8 * u]);
-            const uint32_t pw[4] = {pp.x, pp.y, pp.z, pp.w};
-#pragma unroll
-            for (int c = 0; c < 8; c++)
-                if (8 * u + c < live)  // nothing past the prefix enters a sum
-                    acc[g] = (c & 1) ? fma_mix_hi(pw[c >> 1], vw[c >> 1], acc[g]) : fma_mix_lo(pw[c >> 1], vw[c >> 1], acc[g]);
+    for (int p0 = blockIdx.z * kPos; p0 < n; p0 += step) {
+        __syncthreads();  // the totals are there; the probabilities before are spent
+        for (int i = tid; i < G * kPos; i += NT) {
+            const int g = i / kPos, p = i - g * kPos;
+            ps[g][p] = p0 + p < n
+                           ? (uint16_t)float_to_half_bits(__fdiv_rn(sc[(row0 + g) * S + p0 + p], tot[g]))
+                           : (uint16_t)0;
         }
-    }
+        __syncthreads();
+        const int pr = p0 + r * kRun, live = min(kRun, n - pr);  // the thread's run and its positions
+        if (live > 0) {
+            float acc[G];
 #pragma unroll
-    for (int g = 0; g < G; g++)
-        runs[((row0 + g) * (S / kRun) + pr / kRun) * HD + d] = acc[g];
+            for (int g = 0; g < G; g++)
+                acc[g] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const uint32_t vw[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    const v4u_stream pp = *(const v4u_stream *)(&ps[g][r * kRun + 8 * u]);
+                    const uint32_t pw[4] = {pp.x, pp.y, pp.z, pp.w};
+#pragma unroll
+                    for (int c = 0; c < 8; c++)
+                        if (8 * u + c < live)  // nothing past the prefix enters a sum
+                            acc[g] = (c & 1) ? fma_mix_hi(pw[c >> 1], vw[c >> 1], acc[g])
+                                             : fma_mix_lo(pw[c >> 1], vw[c >> 1], acc[g]);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                runs[((row0 + g) * (S / kRun) + pr / kRun) * HD + d] = acc[g];
+        }
+        if (p0 + step < n)
+            vload(pr + step);
+    }
 }
 
 // grid (heads * HD / 64, tokens), 64 threads: an element's runs in order, a
@@ -241,6 +268,213 @@ __global__ __launch_bounds__(64) void attn_split_finish_kernel(int heads, int hd
     }
 }
 
+// ---- a workgroup a token and a few of its heads ------------------------------
+//
+// grid (heads / GH * HD / VD, tokens), 512 threads: the four steps above in one
+// launch, for GH heads of a key-value head and VD of their elements, over the
+// token's own prefix alone: the scores (a wavefront a block of 64 positions),
+// the exponentials and block sums, the total, then the runs RW at a time,
+// added in order as they come.  Every sum is the split form's, so the two give
+// the same bits.  Scores and exponentials stay in LDS (SLDS) while GH rows of
+// them take at most kRowsLds, else in the caller's rows (which one workgroup
+// writes: VD is HD then).
+// What bounds it: few tokens, one workgroup's chain of steps (about 1 us a 100
+// positions, 0.5 with VD of 32, whose chunks are four times as long); many,
+// the keys and values read once a GH heads.
+constexpr int kRowsThreads = 512;
+constexpr size_t kRowsLds = 32 * 1024;
+
+template <int HD, int GH, int VD, bool SLDS>
+__global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
+    const uint16_t *__restrict__ qh, int heads, int kv_heads, const int32_t *__restrict__ positions, int limit,
+    const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, int context, float scale, int S,
+    int8_t *__restrict__ q, float *__restrict__ scales, int32_t *__restrict__ qsum, float *sc, float *bs,
+    const int32_t *__restrict__ slots, int nslots) {
+    constexpr int NT = kRowsThreads, NW = NT / 64, kPieces = HD / 8;
+    constexpr int RW = NT / VD, kPos = RW * kRun;  // runs and positions a chunk
+    static_assert(SLDS || VD == HD, "the caller's rows have one writer");
+    extern __shared__ __align__(16) float dyn[];  // SLDS: [GH][S] scores, then exponentials; [GH][S / 64] block sums
+    __shared__ __align__(16) v4u_stream qs[GH][kPieces];
+    __shared__ float mw[NW][GH], tot[GH];
+    __shared__ __align__(16) uint16_t ps[2][GH][kPos];
+    __shared__ float rs[2][RW][GH][VD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h0 = blockIdx.x / (HD / VD) * GH, d0 = blockIdx.x % (HD / VD) * VD;
+    const int kvh = h0 / (heads / kv_heads), t = blockIdx.y;
+    const int n = min(positions[t] + 1, limit);
+    const int nb = n > 0 ? (n + kBlock - 1) / kBlock : 0, chunks = n > 0 ? (n + kPos - 1) / kPos : 0;
+    if (slots) {  // reads stay inside the caches
+        const size_t at = (size_t)min(max(slots[t], 0), nslots - 1) * kv_heads * HD * context;
+        kcache += at;
+        vcache += at;
+    }
+    const size_t row0 = (size_t)t * heads + h0;
+    float *s = SLDS ? dyn : sc + row0 * S;
+    float *bsum = SLDS ? dyn + (size_t)GH * S : bs + row0 * (S / kBlock);
+    const int d = tid % VD, r = tid / VD;  // this thread's element and run of a chunk (none past RW)
+    const uint16_t *vrow = vcache + ((size_t)kvh * HD + d0 + d) * context;
+    auto vload = [&](v4u_stream *v, int pr) __attribute__((always_inline)) {  // the run from position pr
+        if (pr < n) {
+#pragma unroll
+            for (int u = 0; u < 4; u++)  // context is a multiple of 8; pieces past the prefix are not used
+                v[u] = *(const v4u_stream *)(vrow + min(pr + 8 * u, context - 8));
+        }
+    };
+    v4u_stream v[4] = {};
+    vload(v, r * kRun);
+    if (tid < GH * kPieces)
+        (&qs[0][0])[tid] = ((const v4u_stream *)(qh + row0 * HD))[tid];
+    __syncthreads();
+
+    // the scores and their maximum
+    float m[GH];
+#pragma unroll
+    for (int g = 0; g < GH; g++)
+        m[g] = -INFINITY;
+    for (int b = wave; b < nb; b += NW) {
+        const int p = b * kBlock + lane;
+        const v4u_stream *kr = (const v4u_stream *)(kcache + (size_t)kvh * HD * context) + min(p, n - 1);
+        v4u_stream k[kPieces];
+#pragma unroll
+        for (int i = 0; i < kPieces; i++)
+            k[i] = kr[(size_t)i * context];
+        asm volatile("" ::: "memory");  // the queries are read here, not kept across the loop (GH of 4: 256 registers)
+#pragma unroll
+        for (int g = 0; g < GH; g++) {
+            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kPieces; i++) {
+                const v4u_stream qq = qs[g][i], kk = k[i];
+                s0 = fma_mix_lo(qq.x, kk.x, s0);
+                s1 = fma_mix_hi(qq.x, kk.x, s1);
+                s2 = fma_mix_lo(qq.y, kk.y, s2);
+                s3 = fma_mix_hi(qq.y, kk.y, s3);
+                s0 = fma_mix_lo(qq.z, kk.z, s0);
+                s1 = fma_mix_hi(qq.z, kk.z, s1);
+                s2 = fma_mix_lo(qq.w, kk.w, s2);
+                s3 = fma_mix_hi(qq.w, kk.w, s3);
+            }
+            const float x = scale * ((s0 + s1) + (s2 + s3));
+            if (p < n) {
+                s[(size_t)g * S + p] = x;
+                m[g] = fmaxf(m[g], x);
+            }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < GH; g++) {
+        m[g] = wave_max(m[g]);
+        if (lane == 0)
+            mw[wave][g] = m[g];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < GH; g++)
+#pragma unroll
+        for (int w = 0; w < NW; w++)
+            m[g] = fmaxf(m[g], mw[w][g]);
+
+    // the exponentials in place (a lane's own scores) and the block sums
+    for (int b = wave; b < nb; b += NW) {
+        const int p = b * kBlock + lane;
+        float df[GH], e[GH];
+#pragma unroll
+        for (int g = 0; g < GH; g++)
+            df[g] = (p < n ? s[(size_t)g * S + p] : m[g]) - m[g];
+        exp_neg_n<GH>(df, e);
+#pragma unroll
+        for (int g = 0; g < GH; g++) {
+            e[g] = p < n ? e[g] : 0.0f;
+            if (p < n)
+                s[(size_t)g * S + p] = e[g];
+            const float sum = wave_pairwise_sum(e[g]);
+            if (lane == 0)
+                bsum[g * (S / kBlock) + b] = sum;
+        }
+    }
+    __syncthreads();
+    // the totals, blocks in order: wavefront g head g's
+    if (wave < GH) {
+        float total = 0.0f;
+        for (int c0 = 0; c0 < nb; c0 += 64) {
+            const float w = bsum[wave * (S / kBlock) + min(c0 + lane, nb - 1)];
+            const int cn = min(64, nb - c0);
+            for (int i = 0; i < cn; i++)
+                total = total + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), i));
+        }
+        if (lane == 0)
+            tot[wave] = total;
+    }
+    __syncthreads();
+
+    // the value sums: a chunk's probabilities, then its runs, added to the
+    // outputs while the next chunk's are taken
+    float o = 0.0f;  // thread g * VD + d: head g's element d
+    const int og = tid / VD;
+    for (int c = 0; c < chunks; c++) {
+        const int buf = c & 1, p0 = c * kPos, pr = p0 + r * kRun;
+        for (int i = tid; i < GH * kPos; i += NT) {
+            const int g = i / kPos, p = i - g * kPos;
+            ps[buf][g][p] = p0 + p < n ? (uint16_t)float_to_half_bits(__fdiv_rn(s[(size_t)g * S + p0 + p], tot[g]))
+                                       : (uint16_t)0;
+        }
+        v4u_stream vn[4] = {};
+        vload(vn, pr + kPos);
+        __syncthreads();
+        if (c > 0 && tid < GH * VD) {
+#pragma unroll
+            for (int i = 0; i < RW; i++)
+                o = o + rs[buf ^ 1][i][og][d];
+        }
+        const int live = r < RW ? min(kRun, n - pr) : 0;  // the run's positions
+        if (live > 0) {
+            float acc[GH];
+#pragma unroll
+            for (int g = 0; g < GH; g++)
+                acc[g] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const uint32_t vw[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int g = 0; g < GH; g++) {
+                    const v4u_stream pp = *(const v4u_stream *)(&ps[buf][g][r * kRun + 8 * u]);
+                    const uint32_t pw[4] = {pp.x, pp.y, pp.z, pp.w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (8 * u + e < live)  // nothing past the prefix enters a sum
+                            acc[g] = (e & 1) ? fma_mix_hi(pw[e >> 1], vw[e >> 1], acc[g])
+                                             : fma_mix_lo(pw[e >> 1], vw[e >> 1], acc[g]);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < GH; g++)
+                rs[buf][r][g][d] = acc[g];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            v[u] = vn[u];
+    }
+    __syncthreads();
+    if (tid < GH * VD) {
+        const int last = chunks - 1, runs = (n - last * kPos + kRun - 1) / kRun;  // of the last chunk
+        if (chunks > 0) {
+#pragma unroll
+            for (int i = 0; i < RW; i++)
+                o = i < runs ? o + rs[last & 1][i][og][d] : o;
+        }
+        // whole 32-lane groups, a Q8_0 block each
+        const int width = heads * HD, col = (h0 + og) * HD + d0 + d;
+        float stored;
+        int32_t sm;
+        const int32_t nq = q8_0_lane(o, &stored, &sm);
+        q[(size_t)t * width + col] = (int8_t)nq;
+        if ((lane & 31) == 0) {
+            scales[(size_t)t * (width >> 5) + (col >> 5)] = stored;
+            qsum[(size_t)t * (width >> 5) + (col >> 5)] = sm;
+        }
+    }
+}
+
 // ---- a prompt ---------------------------------------------------------------
 //
 // grid (heads, ceil(M / 32)), a workgroup per (query head, 32-token tile), NW
@@ -271,7 +505,6 @@ typedef float pl_v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t pl_v2u __attribute__((ext_vector_type(2)));
 
 constexpr int kPlTok = 32;
-constexpr int kPlOne = 1024;  // positions the LDS form takes
 
 template <int HD, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
@@ -289,7 +522,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kPlTok, t = t0 + li;
     // this lane's token's positions (a negative position: as the LDS form to
     // 1024 positions, one; as the serial passes past them, none)
-    const int n = t < M ? max(min(positions[t] + 1, limit), limit <= kPlOne ? 1 : 0) : 0;
+    const int n = t < M ? max(min(positions[t] + 1, limit), limit <= kOne ? 1 : 0) : 0;
     int nmax = n, nmin = t < M ? n : limit;
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) {
@@ -661,62 +894,137 @@ int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, i
     return check_launch("qwen_attention long prompt");
 }
 
-// The runs' floats of up to kSplitTokens tokens, past the scores' workspace.
-constexpr int kSplitTokens = 16;
+static size_t rows_lds(int gh, int S) { return (size_t)gh * (S + S / kBlock) * sizeof(float); }
+
+// Whether a head's elements go 32 a workgroup: while the CUs hold them all.
+static bool rows_sliced(gx_ctx *ctx, int M, int heads, int hd, int S) {
+    return (size_t)M * heads * (hd / 32) <= 2 * (size_t)ctx->cu_count && rows_lds(1, S) <= kRowsLds;
+}
+
+// Which form a call past the one-kernel form's prefixes takes: a workgroup a
+// token's heads, or the positions spread over the chip in four launches.  The
+// launch covers `limit` positions; the tokens may be anywhere below (a step
+// replayed from a graph).  The rows form is the faster for a lone
+// conversation's tokens to 1,024 positions and for many tokens, the split form
+// for few tokens far in.  32 heads of 128, us rows / split at positions 20 /
+// 600 / 1023: one token 7.2 / 14.2, 10.3 / 15.6, 12.4 / 15.2; conversations:
+// eight 7.0 / 14.7, 20.5 / 21.6, 28.7 / 23.5, twelve 7.9 / 14.9, 21 / 24, 29.6
+// / 28.1, 32 10.6 / 28.4, 31 / 51, 44 / 62.  Far in: one token at 4,095 33 /
+// 20, conversations at 2,999 sixteen 83 / 67, 24 131 / 135, 128 420 / 690.
+// (The forms before them: one token in a cache of 1,024 9.2 at 20 and 23 at
+// 1,023; the serial passes 16 and 44 for eight conversations, and 119, 166 and
+// 565 at 2,999 for sixteen, 24 and 128.)
+bool attn_rows_form(gx_ctx *ctx, int M, int heads, int limit, bool slots) {
+    if (M > kSplitTokens)
+        return true;
+    return limit <= kOne && (!slots || (size_t)M * heads > (size_t)ctx->cu_count);
+}
+
+// sc: [M][heads][S] floats, bs: [M][heads][S / 64] floats (used past kRowsLds).
+// Heads a workgroup: as many of a key-value head's as leave the CUs busy (us
+// 1 / 2 / 4 heads, 32 of 128 at 1,024 positions: 16 tokens 45 / 32 / 38, 32
+// tokens 82 / 48 / 44, 128 298 / 169 / 120).
+int launch_attn_rows(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
+                     const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
+                     float scale, int8_t *q, float *scales, int32_t *qsum, float *sc, float *bs, const int32_t *slots,
+                     int nslots) {
+    int gh = std::min(heads / kv_heads, 4);
+    while (gh > 1 && (size_t)M * heads <= (gh == 4 ? 3 : 1) * (size_t)ctx->cu_count)
+        gh /= 2;
+    const size_t lds = rows_lds(gh, S);
+    const bool sliced = gh == 1 && rows_sliced(ctx, M, heads, hd, S);
+#define GX_ROWS(HH, GG, VV, LL)                                                                                      \
+    attn_rows_kernel<HH, GG, VV, LL>                                                                                 \
+        <<<dim3((unsigned)(heads / GG * (HH / VV)), (unsigned)M), kRowsThreads, LL ? lds : 0, ctx->stream>>>(        \
+            qh, heads, kv_heads, positions, limit, kcache, vcache, context, scale, S, q, scales, qsum, sc, bs,       \
+            slots, nslots)
+#define GX_ROWS_G(HH, GG)                                                                                            \
+    do {                                                                                                             \
+        if (lds <= kRowsLds)                                                                                         \
+            GX_ROWS(HH, GG, HH, true);                                                                               \
+        else                                                                                                         \
+            GX_ROWS(HH, GG, HH, false);                                                                              \
+    } while (0)
+#define GX_ROWS_H(HH)                                                                                                \
+    do {                                                                                                             \
+        if (sliced)                                                                                                  \
+            GX_ROWS(HH, 1, 32, true);                                                                                \
+        else if (gh == 1)                                                                                            \
+            GX_ROWS_G(HH, 1);                                                                                        \
+        else if (gh == 2)                                                                                            \
+            GX_ROWS_G(HH, 2);                                                                                        \
+        else                                                                                                         \
+            GX_ROWS_G(HH, 4);                                                                                        \
+    } while (0)
+    if (hd == 32)
+        GX_ROWS_H(32);
+    else if (hd == 64)
+        GX_ROWS_H(64);
+    else if (hd == 96)
+        GX_ROWS_H(96);
+    else
+        GX_ROWS_H(128);
+#undef GX_ROWS_H
+#undef GX_ROWS_G
+#undef GX_ROWS
+    return check_launch("qwen_attention rows");
+}
+
+// The runs' floats, past the scores' workspace.
 size_t attn_split_workspace(int M, int heads, int S) {
     return (size_t)std::min(M, kSplitTokens) * heads * (S / kRun) * 128 * sizeof(float);
 }
 
-// sc: [M][heads][S] floats; small: as many halves (the block maxima and sums
-// take an eighth of a half a position); runs: attn_split_workspace bytes.
+// A step's workgroups along the prefix: one a piece while their wavefronts
+// (`others` a piece) number at most kSplitWaves, past that each takes several.
+// So a step replayed for a long context does not pay for its empty workgroups:
+// eight conversations of 32 heads at position 100, launched for 16,384, 31 ->
+// 16 us, at position 16,383 231 -> 223.
+static int split_share(int pieces, int others) { return std::min(pieces, std::max(1, kSplitWaves / others)); }
+
+// M <= kSplitTokens.  sc: [M][heads][S] floats; small: as many halves (the
+// block maxima and sums take an eighth of a half a position); runs:
+// attn_split_workspace bytes.
 int launch_attn_split(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
                       const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                       float scale, int8_t *q, float *scales, int32_t *qsum, float *sc, float *small, float *runs,
                       const int32_t *slots, int nslots) {
     const int G = heads / kv_heads, width = heads * hd;
-    float *mx = small, *bs = small + (size_t)std::min(M, kSplitTokens) * heads * (S / kBlock);
-    const int nblocks = (limit + kBlock - 1) / kBlock;
-    for (int t0 = 0; t0 < M; t0 += kSplitTokens) {
-        const unsigned tn = (unsigned)std::min(kSplitTokens, M - t0);
-        const uint16_t *qt = qh + (size_t)t0 * width;
-        const int32_t *pos = positions + t0, *sl = slots ? slots + t0 : nullptr;
-        const int rw = 256 / hd, pw = rw * kRun;
-        const dim3 vgrid((unsigned)kv_heads, (unsigned)((limit + pw - 1) / pw), tn);
+    float *mx = small, *bs = small + (size_t)M * heads * (S / kBlock);
+    const int nblocks = (limit + kBlock - 1) / kBlock, pw = 256 / hd * kRun, vx = heads / std::min(G, 4);
+    const dim3 sgrid((unsigned)kv_heads, (unsigned)M, (unsigned)split_share(nblocks, heads * M));
+    const dim3 egrid((unsigned)heads, (unsigned)M, (unsigned)split_share((nblocks + 3) / 4, 4 * heads * M));
+    const dim3 vgrid((unsigned)vx, (unsigned)M, (unsigned)split_share((limit + pw - 1) / pw, 4 * vx * M));
 #define GX_SPLIT_V(HH, GG)                                                                                           \
     attn_split_values_kernel<HH, GG><<<vgrid, (256 / HH) * HH, 0, ctx->stream>>>(                                    \
-        heads, kv_heads, pos, limit, vcache, context, S, sc, bs, runs, sl, nslots)
+        heads, kv_heads, positions, limit, vcache, context, S, sc, bs, runs, slots, nslots, (int)vgrid.z)
 #define GX_SPLIT(HH)                                                                                                 \
     do {                                                                                                             \
-        attn_split_scores_kernel<HH><<<dim3((unsigned)kv_heads, (unsigned)nblocks, tn), 64 * G, 0, ctx->stream>>>(   \
-            qt, heads, kv_heads, pos, limit, kcache, context, scale, S, sc, mx, sl, nslots);                         \
-        attn_split_exp_kernel<<<dim3((unsigned)((nblocks + 3) / 4), (unsigned)heads, tn), 256, 0, ctx->stream>>>(    \
-            heads, pos, limit, S, sc, mx, bs);                                                                       \
+        attn_split_scores_kernel<HH><<<sgrid, 64 * G, 0, ctx->stream>>>(qh, heads, kv_heads, positions, limit,       \
+                                                                        kcache, context, scale, S, sc, mx, slots,    \
+                                                                        nslots, (int)sgrid.z);                       \
+        attn_split_exp_kernel<<<egrid, 256, 0, ctx->stream>>>(heads, kv_heads, positions, limit, S, sc, mx, bs,      \
+                                                              (int)egrid.z);                                         \
         if (G == 1)                                                                                                  \
             GX_SPLIT_V(HH, 1);                                                                                       \
         else if (G == 2)                                                                                             \
             GX_SPLIT_V(HH, 2);                                                                                       \
-        else if (G == 4)                                                                                             \
-            GX_SPLIT_V(HH, 4);                                                                                       \
         else                                                                                                         \
-            GX_SPLIT_V(HH, 8);                                                                                       \
+            GX_SPLIT_V(HH, 4);                                                                                       \
     } while (0)
-        if (hd == 32)
-            GX_SPLIT(32);
-        else if (hd == 64)
-            GX_SPLIT(64);
-        else if (hd == 96)
-            GX_SPLIT(96);
-        else
-            GX_SPLIT(128);
+    if (hd == 32)
+        GX_SPLIT(32);
+    else if (hd == 64)
+        GX_SPLIT(64);
+    else if (hd == 96)
+        GX_SPLIT(96);
+    else
+        GX_SPLIT(128);
 #undef GX_SPLIT
 #undef GX_SPLIT_V
-        attn_split_finish_kernel<<<dim3((unsigned)((width + 63) / 64), tn), 64, 0, ctx->stream>>>(
-            heads, hd, pos, limit, S, runs, q + (size_t)t0 * width, scales + (size_t)t0 * (width >> 5),
-            qsum + (size_t)t0 * (width >> 5));
-        if (int rc = check_launch("qwen_attention split"))
-            return rc;
-    }
-    return GX_OK;
+    attn_split_finish_kernel<<<dim3((unsigned)((width + 63) / 64), (unsigned)M), 64, 0, ctx->stream>>>(
+        heads, hd, positions, limit, S, runs, q, scales, qsum);
+    return check_launch("qwen_attention split");
 }
 
 }  // namespace gx

@@ -177,6 +177,11 @@ bool attn_prompt_long_fits(int hd, int limit, int context);
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                             float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f);
+bool attn_rows_form(gx_ctx *ctx, int M, int heads, int limit, bool slots);
+int launch_attn_rows(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
+                     const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
+                     float scale, int8_t *q, float *scales, int32_t *qsum, float *sc, float *bs, const int32_t *slots,
+                     int nslots);
 size_t attn_split_workspace(int M, int heads, int S);
 int launch_attn_split(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit, int S,
                       const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,

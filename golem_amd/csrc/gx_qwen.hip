@@ -2268,13 +2268,17 @@ int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int
     if (parallel && (M <= 4 || slots) && limit <= kDecodeMax)
         return launch_par<false>(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context, scale,
                                  q, scales, qsum, slots, nslots, QkRope{}, heads_f);
-    // Longer prefixes: the same order, the positions spread over the chip.
-    // (One position of 32 heads at 3,000: 104 us in the serial passes.)
-    if (parallel && (M <= 4 || slots) && !heads_f && workspace_bytes >= qwen_attention_workspace(M, heads, max_pos))
+    // Longer prefixes: the same order, a workgroup a token's heads or the
+    // positions spread over the chip.
+    if (parallel && (M <= 4 || slots) && !heads_f && workspace_bytes >= qwen_attention_workspace(M, heads, max_pos)) {
+        if (attn_rows_form(ctx, M, heads, limit, slots != nullptr))
+            return launch_attn_rows(ctx, qh, M, heads, kv_heads, hd, limit, S, positions, kcache, vcache, context,
+                                    scale, q, scales, qsum, sc, (float *)prob, slots, nslots);
         return launch_attn_split(ctx, qh, M, heads, kv_heads, hd, limit, S, positions, kcache, vcache, context, scale,
                                  q, scales, qsum, sc, (float *)prob,
                                  (float *)(workspace + qwen_attention_workspace_least(M, heads, max_pos)), slots,
                                  nslots);
+    }
     // A prompt of one conversation in the parallel order: the matrix cores,
     // the scores in LDS while two workgroups a CU hold them (576 positions)
     // or the tiles are few, in three sweeps past that.  32 heads of 128 (us,

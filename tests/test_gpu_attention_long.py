@@ -89,15 +89,16 @@ def test_long_decode_is_the_parallel_order(dev, orc, hd, heads, kv, positions):
 
 
 def test_long_decode_of_many_conversations(dev, orc):
-    """Eighteen tokens of three conversations (more than the split form holds
-    at once), a slot out of range (read inside the caches), a negative
-    position (nothing visible: zeros); with the serial passes' workspace alone
-    the call runs them."""
+    """Eighteen tokens of three conversations (more than the split form takes),
+    two slots out of range (read inside the caches), a negative position
+    (nothing visible: zeros); with the serial passes' workspace alone the call
+    runs them."""
     hd, heads, kv, nslots, n, context = 64, 4, 2, 3, 800, 808
     g = synth.rng(5)
     k, v, kt, vt = _caches(g, nslots, n, kv, hd, context, False)
     pos = np.array([799, 0, -1, 64, 700, 31, 32, 767, 768, 5, 63, 127, 128, 400, 798, 255, 256, 511], np.int32)
     slots = np.array([i % 3 for i in range(18)], np.int32)
+    slots[4], slots[10] = nslots + 2, -1
     qf = (g.standard_normal((18, heads * hd)) * 1.5).astype(np.float16)
     read = np.clip(slots, 0, nslots - 1)
     q8, sc, qs = _run(dev, "gx_qwen_attention_parallel", qf, pos, kt, vt, heads, kv, hd, n - 1, context, slots, nslots)
@@ -110,6 +111,36 @@ def test_long_decode_of_many_conversations(dev, orc):
     for a, b in zip(serial, least):
         np.testing.assert_array_equal(a, b)
     assert (q8[2] == 0).all() and (sc[2] == 0).all() and (serial[0][2] == 0).all()
+
+
+# head width, heads, key-value heads, tokens, longest prefix.  A workgroup a
+# token's heads: one, two and four heads each, their scores in LDS and (past
+# 2,016 positions of four heads, 4,032 of two, 8,064 of one) in the caller's
+# rows; a head's elements 32 a workgroup.  The positions over the chip: a
+# workgroup a piece, and several pieces a workgroup
+FORMS = [(128, 8, 1, 20, 900), (64, 16, 4, 20, 800), (32, 16, 8, 20, 4100), (128, 32, 8, 28, 800),
+         (96, 32, 8, 26, 2310), (64, 2, 1, 17, 8200), (96, 4, 4, 3, 1000), (64, 32, 8, 16, 1024), (128, 32, 8, 8, 1000),
+         (64, 8, 1, 16, 1100), (32, 32, 32, 16, 2400)]
+
+
+@pytest.mark.parametrize("hd,heads,kv,M,n", FORMS)
+def test_long_decode_forms(dev, orc, hd, heads, kv, M, n):
+    """Bit for bit the restated order in either form, over prefixes of no
+    position, one, the edges of runs, blocks and chunks, all; slots out of
+    range read inside the caches."""
+    g = synth.rng(hd + M + n)
+    nslots, context = 2, (n + 7) // 8 * 8
+    edges = [n - 1, -1, 0, 31, 32, 63, 64, 127, 128, 159, 160, 255, 256, 511, 512, 575, 576, n // 2, n - 33, n - 64]
+    pos = np.array([edges[i] if i < len(edges) else int(g.integers(0, n)) for i in range(M)], np.int32)
+    slots = np.array([nslots + 5 if i == 3 else -2 if i == 2 else i % nslots for i in range(M)], np.int32)
+    k, v, kt, vt = _caches(g, nslots, n, kv, hd, context, False)
+    qf = (g.standard_normal((M, heads * hd)) * 1.5).astype(np.float16)
+    read = np.clip(slots, 0, nslots - 1)
+    q8, sc, qs = _run(dev, "gx_qwen_attention_parallel", qf, pos, kt, vt, heads, kv, hd, n - 1, context, slots, nslots)
+    want = orc.Batch(_oracle(orc, "orc_attend_parallel", qf, k, v, pos, read, range(M), heads, kv, hd)).quantize()
+    np.testing.assert_array_equal(q8, want.q_rows())
+    np.testing.assert_array_equal(_bits(sc), _bits(want.scales_rows()))
+    np.testing.assert_array_equal(qs, want.qsum_rows())
 
 
 # head width, heads, key-value heads, M, first position, context: few tiles
