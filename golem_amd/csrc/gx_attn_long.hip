@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
     const uint16_t *__restrict__ qh, int heads, int kv_heads, const int32_t *__restrict__ positions, int limit,
     const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, int context, float scale, int S,
     int8_t *__restrict__ q, float *__restrict__ scales, int32_t *__restrict__ qsum, float *sc, float *bs,
-    const int32_t *__restrict__ slots, int nslots) {
+    const int32_t *__restrict__ slots, int nslots, int least) {
     constexpr int NT = kRowsThreads, NW = NT / 64, kPieces = HD / 8;
     constexpr int RW = NT / VD, kPos = RW * kRun;  // runs and positions a chunk
     static_assert(SLDS || VD == HD, "the caller's rows have one writer");
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h0 = blockIdx.x / (HD / VD) * GH, d0 = blockIdx.x % (HD / VD) * VD;
     const int kvh = h0 / (heads / kv_heads), t = blockIdx.y;
-    const int n = min(positions[t] + 1, limit);
+    const int n = max(min(positions[t] + 1, limit), least);
     const int nb = n > 0 ? (n + kBlock - 1) / kBlock : 0, chunks = n > 0 ? (n + kPos - 1) / kPos : 0;
     if (slots) {  // reads stay inside the caches
         const size_t at = (size_t)min(max(slots[t], 0), nslots - 1) * kv_heads * HD * context;
@@ -933,11 +933,14 @@ int launch_attn_rows(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_h
         gh /= 2;
     const size_t lds = rows_lds(gh, S);
     const bool sliced = gh == 1 && rows_sliced(ctx, M, heads, hd, S);
+    // A negative position sees one position in a lone conversation's calls to
+    // 1,024 positions, as a prompt's does there, and none in the others.
+    const int least = !slots && limit <= kOne ? 1 : 0;
 #define GX_ROWS(HH, GG, VV, LL)                                                                                      \
     attn_rows_kernel<HH, GG, VV, LL>                                                                                 \
         <<<dim3((unsigned)(heads / GG * (HH / VV)), (unsigned)M), kRowsThreads, LL ? lds : 0, ctx->stream>>>(        \
             qh, heads, kv_heads, positions, limit, kcache, vcache, context, scale, S, q, scales, qsum, sc, bs,       \
-            slots, nslots)
+            slots, nslots, least)
 #define GX_ROWS_G(HH, GG)                                                                                            \
     do {                                                                                                             \
         if (lds <= kRowsLds)                                                                                         \

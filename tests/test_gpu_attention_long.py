@@ -113,6 +113,24 @@ def test_long_decode_of_many_conversations(dev, orc):
     assert (q8[2] == 0).all() and (sc[2] == 0).all() and (serial[0][2] == 0).all()
 
 
+@pytest.mark.parametrize("M,n", [(2, 900), (4, 1024), (2, 1100)])
+def test_negative_positions_of_a_lone_conversation(dev, orc, M, n):
+    """To 1,024 positions a negative position sees the first one (as a prompt's
+    does), past them none: zeros."""
+    hd, heads, kv = 64, 4, 2
+    context = (n + 7) // 8 * 8
+    g = synth.rng(M + n)
+    pos = np.array([n - 1, -1, -3, 0][:M], np.int32)
+    k, v, kt, vt = _caches(g, 1, n, kv, hd, context, False)
+    qf = g.standard_normal((M, heads * hd)).astype(np.float16)
+    q8, sc, qs = _run(dev, "gx_qwen_attention_parallel", qf, pos, kt, vt, heads, kv, hd, n - 1, context)
+    seen = np.maximum(pos, 0) if n <= 1024 else pos
+    want = orc.Batch(_oracle(orc, "orc_attend_parallel", qf, k, v, seen, None, range(M), heads, kv, hd)).quantize()
+    np.testing.assert_array_equal(q8, want.q_rows())
+    np.testing.assert_array_equal(_bits(sc), _bits(want.scales_rows()))
+    np.testing.assert_array_equal(qs, want.qsum_rows())
+
+
 # head width, heads, key-value heads, tokens, longest prefix.  A workgroup a
 # token's heads: one, two and four heads each, their scores in LDS and (past
 # 2,016 positions of four heads, 4,032 of two, 8,064 of one) in the caller's
