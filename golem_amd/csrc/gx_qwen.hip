@@ -1729,11 +1729,12 @@ __global__ __launch_bounds__(kPmThreads, 4) void attn_prompt_mfma_kernel(
     static_assert(HD % 32 == 0, "whole 32-element head blocks");
     constexpr int KS = HD / 16;  // the head in MFMA k-steps
     extern __shared__ __align__(16) float sl[];  // [kPmTok][stride]: scores, then exponentials
-    __shared__ int nrow[kPmTok];
+    __shared__ int nrow[kPmTok], nends[2];
     __shared__ float mrow[kPmTok], trow[kPmTok];
     __shared__ float bsum[kPmTok][kPmMax / 64];
     __shared__ __align__(16) uint16_t qs[kPmTok][HD + 8];  // the tile's queries (+8: rows 4 banks apart)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, g = lane >> 5;
     // the second half of the heads takes the token tiles in reverse order:
     // workgroups L and L + grid / 2, which tend to share a CU, then hold
     // tiles i and n - 1 - i (light with heavy) rather than the same tile
@@ -1750,13 +1751,18 @@ __global__ __launch_bounds__(kPmThreads, 4) void attn_prompt_mfma_kernel(
         *(v4u_stream *)&qs[tk][8 * c] =
             *(const v4u_stream *)(qh + ((size_t)min(t0 + tk, M - 1) * heads + h) * HD + 8 * c);
     }
-    if (tid < kPmTok)
-        nrow[tid] = t0 + tid < M ? min(max(positions[t0 + tid], 0) + 1, limit) : 0;
+    if (wave == 0) {
+        const bool has = li == lane && t0 + lane < M;
+        const int n = has ? min(max(positions[t0 + lane], 0) + 1, limit) : 0;
+        if (lane < kPmTok)
+            nrow[lane] = n;
+        // the most and the least of the tokens there are (at most kPmMax: exact as floats)
+        const float most = wave_max((float)n), least = -wave_max(has ? -(float)n : -(float)limit);
+        if (lane == 0)
+            nends[0] = (int)most, nends[1] = (int)least;
+    }
     lds_barrier();
-    int nmax = 0;
-#pragma unroll 8
-    for (int r = 0; r < kPmTok; r++)
-        nmax = max(nmax, nrow[r]);
+    const int nmax = __builtin_amdgcn_readfirstlane(nends[0]), nmin = __builtin_amdgcn_readfirstlane(nends[1]);
     const int np = (nmax + 63) & ~63;  // whole 64-position blocks
 
     // scores: wavefront w takes the 32-position tiles w, w + 4, ...; key
@@ -1901,8 +1907,12 @@ __global__ __launch_bounds__(kPmThreads, 4) void attn_prompt_mfma_kernel(
 
     // values: the probabilities as the row operand, the value pieces as the
     // column operand; piece i + kPmPre is requested as piece i is used
+    // An infinite or NaN value past some token's own positions would reach it
+    // as 0 * inf: such values enter the product as zeros, and each token that
+    // sees them takes them afterwards.
     const uint16_t *pr = (const uint16_t *)(sl + li * stride) + 8 * g;
     pm_v16f acc = {};
+    uint32_t wild = 0;
     if (pv) {
         for (int i0 = i_lo; i0 < i_hi; i0 += kPmPre) {
 #pragma unroll
@@ -1921,9 +1931,33 @@ __global__ __launch_bounds__(kPmThreads, 4) void attn_prompt_mfma_kernel(
                             vv[k] &= keep;
                         }
                     }
+                    if (16 * i + 16 > nmin) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            // an exponent of all ones carries into the half's sign place
+                            const uint32_t f = ((vv[k] & 0x7FFF7FFFu) + 0x04000400u) & 0x80008000u;
+                            wild |= f;
+                            vv[k] &= ~((f >> 15) * 0xFFFFu);
+                        }
+                    }
                     const pm_v8h ap = *(const pm_v8h *)(pr + 16 * i);
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ap, __builtin_bit_cast(pm_v8h, vv), acc, 0, 0, 0);
                 }
+            }
+        }
+    }
+    if (__ballot(wild != 0) != 0) {
+#pragma unroll 1
+        for (int p = max(16 * i_lo, nmin & ~15); p < min(16 * i_hi, nmax); p++) {
+            const uint16_t x = vrow[p];  // this lane's element
+            if ((x & 0x7C00u) != 0x7C00u)
+                continue;
+            const float v = (float)__builtin_bit_cast(_Float16, x);
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int r = 8 * (e >> 2) + 4 * g + (e & 3);
+                const float w = (float)__builtin_bit_cast(_Float16, ((const uint16_t *)(sl + r * stride))[p]);
+                acc[e] = p < nrow[r] ? fmaf(w, v, acc[e]) : acc[e];
             }
         }
     }
