@@ -2313,13 +2313,25 @@ int launch_qwen_attention(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int
                                  (float *)(workspace + qwen_attention_workspace_least(M, heads, max_pos)), slots,
                                  nslots);
     }
-    // A prompt of one conversation in the parallel order: the matrix cores,
-    // the scores in LDS while two workgroups a CU hold them (576 positions)
-    // or the tiles are few, in three sweeps past that.  32 heads of 128 (us,
-    // LDS / sweeps): 512 tokens 26 / 39, 300 after 500 54 / 53, 64 after 900
-    // 39 / 34, 8 after 900 25 / 33, 1000 tokens 135 / 78.
-    const bool sweeps = !slots && M > 4 && attn_prompt_long_fits(hd, limit, context) &&
-                        (limit > kPmMax || (limit > 576 && (size_t)((M + kPmTok - 1) / kPmTok) * heads > 32));
+    // A prompt of one conversation in the parallel order: the matrix cores, the
+    // scores in LDS or, past 1,024 positions and where it is the faster, in
+    // three sweeps.  Past 576 positions the LDS form's workgroups go one a CU,
+    // whatever the head's width, which is what the sweeps cost by: heads of 32
+    // take them but for the fewest tiles, wider ones where the LDS form needs
+    // a second round, those of 96 and 128 only with half of the tokens early
+    // in the prefix (of 128 to eleven blocks, two uneven rounds of a sweep's
+    // eight wavefronts, three quarters, or more than three rounds).  us LDS /
+    // sweeps: 32 heads of 32: 57 tokens to 577 26 / 22, 300 to 1,000 62 / 35;
+    // of 64: 210 to 700 26 / 29, 307 to 1,024 59 / 49; of 128: 128 to 1,024 39
+    // / 45, 300 to 640 47 / 52, 489 to 700 54 / 59, 480 to 600 50 / 46, 300 to
+    // 1,024 68 / 78, 560 to 800 71 / 62, 1,000 to 1,000 135 / 84; 64 heads of
+    // 128: 8 to 1,024 26 / 42, 403 to 577 75 / 66, 540 to 900 131 / 118.
+    const size_t groups = (size_t)((M + kPmTok - 1) / kPmTok) * heads;
+    const size_t cus = (size_t)ctx->cu_count, m = (size_t)M, end = (size_t)limit;
+    const bool early = 2 * m >= end && (hd == 96 || limit > 704 || 4 * m >= 3 * end || groups > 3 * cus);
+    const bool faster = hd == 32 ? groups > 32 : groups > cus && (hd == 64 || early);
+    const bool sweeps =
+        !slots && M > 4 && attn_prompt_long_fits(hd, limit, context) && (limit > kPmMax || (limit > 576 && faster));
     if (parallel && sweeps)
         return launch_attn_prompt_long(ctx, qh, M, heads, kv_heads, hd, limit, positions, kcache, vcache, context,
                                        scale, q, scales, qsum, heads_f);

@@ -189,7 +189,7 @@ def test_long_prompt_on_exact_scores(dev, orc, hd, heads, kv, M, start, context)
     np.testing.assert_array_equal(qs, q8.reshape(M, -1, 32).astype(np.int32).sum(2))
 
 
-@pytest.mark.parametrize("hd,start", [(128, 1100), (64, 600), (128, 0), (64, 300), (96, 505)])
+@pytest.mark.parametrize("hd,start", [(128, 1100), (64, 600), (128, 0), (64, 300), (96, 505), (32, 700)])
 def test_long_prompt_keeps_later_infinities_out(dev, hd, start):
     """An infinite and a NaN value of two tokens in mid-tile: the tokens before
     them get the bits they get without them, the tokens after them everywhere
