@@ -9,6 +9,7 @@
 // summed pairwise and the blocks added in order, the probabilities divided
 // and rounded through fp16, the value sums.
 #include <algorithm>
+#include <type_traits>
 
 #include "gx_device.hpp"
 #include "gx_internal.hpp"
@@ -495,8 +496,8 @@ __global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
 // probabilities and values), the scores and exponentials computed again each
 // time: both cost less than writing them out and reading them back (1,500
 // tokens of 32 heads: 144 MB).  The keys, 32 KB a wavefront's block, come
-// from the L2.  The wavefronts' value sums are added pairwise at the end
-// (w + NW/2, then w + NW/4, ...).
+// from the L2.  The value sums of the eight groups of blocks (b % 8) are added
+// pairwise at the end (c + 4, then c + 2, c + 1).
 // What bounds it: the exponentials (float64, twice) and the MFMAs, about 900
 // and 300 cycles a 32 x 32 tile and sweep.  1,500 tokens of 32 heads: 172 us,
 // where the serial passes took 679 (scores 226, softmax 132, values 321).
@@ -505,14 +506,17 @@ typedef float pl_v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t pl_v2u __attribute__((ext_vector_type(2)));
 
 constexpr int kPlTok = 32;
+constexpr int kPlGroups = 8;  // blocks b with the same b % 8 make one value sum
 
 template <int HD, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
+__global__ __launch_bounds__(64 * NW, HD <= 64 ? 4 : 2) void attn_prompt_long_kernel(
     const uint16_t *__restrict__ qh, int M, int heads, int kv_heads, const int32_t *__restrict__ positions,
     int limit, const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, int context, float scale,
     int8_t *__restrict__ q, float *__restrict__ scales, int32_t *__restrict__ qsum, float *__restrict__ heads_f) {
     constexpr int KS = HD / 16, DB = HD / 32;
-    extern __shared__ __align__(16) float sl[];  // block sums [blocks][32]; at the end the value sums and the output tile
+    using Own = std::integral_constant<int, NW>;
+    using Group = std::integral_constant<int, kPlGroups>;
+    extern __shared__ __align__(16) float sl[];  // block sums [blocks][32]; then the value sums and the output tile
     __shared__ float mw[NW][kPlTok];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, g = lane >> 5;
@@ -560,19 +564,20 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     // the lane's e-th position of a tile is 8 (e / 4) + 4 g + e % 4 in: below `own` = left(first position, end) or not
     auto left = [&](int p0, int end) __attribute__((always_inline)) { return end - p0 - 4 * g; };
     auto in = [](int own, int e) __attribute__((always_inline)) { return 8 * (e >> 2) + (e & 3) < own; };
-    // every tile of this wavefront's blocks: f(first position, scores), the
+    // every tile of blocks b0, b0 + step, ..: f(first position, scores), the
     // next tile's keys on their way
-    auto sweep = [&](auto &&f) __attribute__((always_inline)) {
+    auto sweep = [&](int b0, auto step_tag, auto &&f) __attribute__((always_inline)) {
+        constexpr int step = decltype(step_tag)::value;
         pl_v8h k[KS];
-        if (wave < nb)
-            kload(wave * kBlock, k);
-        for (int b = wave; b < nb; b += NW) {
+        if (b0 < nb)
+            kload(b0 * kBlock, k);
+        for (int b = b0; b < nb; b += step) {
 #pragma unroll
             for (int hf = 0; hf < 2; hf++) {
                 const int p0 = b * kBlock + 32 * hf;
                 float s[16];
                 score(k, s);
-                kload(hf ? (b + NW < nb ? (b + NW) * kBlock : p0) : p0 + 32, k);
+                kload(hf ? (b + step < nb ? (b + step) * kBlock : p0) : p0 + 32, k);
                 f(p0, s, hf);
             }
         }
@@ -580,7 +585,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
 
     // the maximum
     float m = -INFINITY;
-    sweep([&](int p0, const float *s, int) __attribute__((always_inline)) {
+    sweep(wave, Own{}, [&](int p0, const float *s, int) __attribute__((always_inline)) {
         if (p0 + 32 <= nmin) {
 #pragma unroll
             for (int e = 0; e < 16; e++)
@@ -624,7 +629,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     // lane, eight with lane ^ 32, sixteen and thirty-two within the lane, the
     // block's two tiles
     float half_sum = 0.0f;
-    sweep([&](int p0, const float *s, int hf) __attribute__((always_inline)) {
+    sweep(wave, Own{}, [&](int p0, const float *s, int hf) __attribute__((always_inline)) {
         float e16[16], c4[4];
         exps(p0, s, e16);
 #pragma unroll
@@ -688,111 +693,136 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     // 0 * inf: the wavefront's tiles from the first with such a value past
     // some token's own positions wait.  (Looked for ahead of the sweep: in it,
     // where the values are at hand, it spilled, 172 -> 186 us.)
-    int late = nmax;
-    int b0 = wave;
-    while (b0 < nb && (b0 + 1) * kBlock <= nmin)
-        b0 += NW;
+    //
+    // The value sums go by eight groups of blocks whatever the wavefronts, so
+    // that a token's bits do not depend on the batch it came in: of four
+    // wavefronts each takes its upper group first and leaves that sum in LDS.
+    float *upper = sl + (size_t)wave * DB * 16 * 64 + lane;
+    __syncthreads();  // the block sums are spent
 #pragma unroll 1
-    for (int p0 = b0 * kBlock; p0 < late; p0 += (p0 & 32) ? NW * kBlock - 32 : 32) {
-        const int own = left(p0, nmax);
-        uint32_t any = 0;
-#pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int w = 0; w < 8; w++) {
-                const int e = 2 * w;
-                const uint32_t keep = (in(own, e) ? 0x7FFFu : 0u) | (in(own, e + 1) ? 0x7FFF0000u : 0u);
-                // an exponent of all ones carries into the half's sign place
-                any |= ((vload(p0, db, w >> 2, (w >> 1) & 1)[w & 1] & keep) + 0x04000400u) & 0x80008000u;
-            }
-        if (p0 + 32 > nmin && __ballot(any != 0) != 0)
-            late = p0;
-    }
-    late = __builtin_amdgcn_readfirstlane(late);
-    sweep([&](int p0, const float *s, int) __attribute__((always_inline)) {
-        if (p0 >= late)
-            return;
-        pl_v2u v[DB][2][2];  // [element block][k-step][positions 4 g .., 8 + 4 g ..]
-#pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int st = 0; st < 2; st++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-                    v[db][st][u] = vload(p0, db, st, u);
-        uint32_t ph[8];
-        probs(p0, s, ph);
-        if (p0 + 32 > nmax) {  // values past the tile's last position may be unwritten: zeros
+    for (int group = wave + kPlGroups - NW; group >= 0; group -= NW) {
+        int late = nmax;
+        int b0 = group;
+        while (b0 < nb && (b0 + 1) * kBlock <= nmin)
+            b0 += kPlGroups;
+#pragma unroll 1
+        for (int p0 = b0 * kBlock; p0 < late; p0 += (p0 & 32) ? kPlGroups * kBlock - 32 : 32) {
             const int own = left(p0, nmax);
+            uint32_t any = 0;
 #pragma unroll
-            for (int st = 0; st < 2; st++)
+            for (int db = 0; db < DB; db++)
 #pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int c = 0; c < 2; c++) {
-                        const int e = 8 * st + 4 * u + 2 * c;
-                        const uint32_t keep = (in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u);
-#pragma unroll
-                        for (int db = 0; db < DB; db++)
-                            v[db][st][u][c] &= keep;
-                    }
+                for (int w = 0; w < 8; w++) {
+                    const int e = 2 * w;
+                    const uint32_t keep = (in(own, e) ? 0x7FFFu : 0u) | (in(own, e + 1) ? 0x7FFF0000u : 0u);
+                    // an exponent of all ones carries into the half's sign place
+                    any |= ((vload(p0, db, w >> 2, (w >> 1) & 1)[w & 1] & keep) + 0x04000400u) & 0x80008000u;
+                }
+            if (p0 + 32 > nmin && __ballot(any != 0) != 0)
+                late = p0;
         }
+        late = __builtin_amdgcn_readfirstlane(late);
+        sweep(group, Group{}, [&](int p0, const float *s, int) __attribute__((always_inline)) {
+            if (p0 >= late)
+                return;
+            pl_v2u v[DB][2][2];  // [element block][k-step][positions 4 g .., 8 + 4 g ..]
 #pragma unroll
-        for (int st = 0; st < 2; st++) {
-            const uint4 pb = make_uint4(ph[4 * st], ph[4 * st + 1], ph[4 * st + 2], ph[4 * st + 3]);
+            for (int db = 0; db < DB; db++)
 #pragma unroll
-            for (int db = 0; db < DB; db++) {
-                const uint4 va = make_uint4(v[db][st][0].x, v[db][st][0].y, v[db][st][1].x, v[db][st][1].y);
-                acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pl_v8h, va),
-                                                                 __builtin_bit_cast(pl_v8h, pb), acc[db], 0, 0, 0);
-            }
-        }
-    });
-
-    // the tiles that waited, a token at a time with the values past it zeroed
-#pragma unroll 1
-    for (int p0 = late; p0 < nmax; p0 += (p0 & 32) ? NW * kBlock - 32 : 32) {
-        uint32_t ph[8];
-        {
-            pl_v8h k[KS];
-            float s[16];
-            kload(p0, k);
-            score(k, s);
+                for (int st = 0; st < 2; st++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        v[db][st][u] = vload(p0, db, st, u);
+            uint32_t ph[8];
             probs(p0, s, ph);
-        }
-#pragma unroll 1
-        for (int tt = 0; tt < kPlTok; tt++) {
-            const int own = left(p0, __builtin_amdgcn_readlane(n, tt));
+            if (p0 + 32 > nmax) {  // values past the tile's last position may be unwritten: zeros
+                const int own = left(p0, nmax);
 #pragma unroll
-            for (int db = 0; db < DB; db++) {
-                pl_v16f one = acc[db];
+                for (int st = 0; st < 2; st++)
 #pragma unroll
-                for (int st = 0; st < 2; st++) {
-                    uint32_t vm[4];
-#pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        const pl_v2u x = vload(p0, db, st, u);
+                    for (int u = 0; u < 2; u++)
 #pragma unroll
                         for (int c = 0; c < 2; c++) {
                             const int e = 8 * st + 4 * u + 2 * c;
-                            vm[2 * u + c] =
-                                x[c] & ((in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u));
-                        }
-                    }
-                    const uint4 pb = make_uint4(ph[4 * st], ph[4 * st + 1], ph[4 * st + 2], ph[4 * st + 3]);
-                    const uint4 va = make_uint4(vm[0], vm[1], vm[2], vm[3]);
-                    one = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pl_v8h, va),
-                                                                 __builtin_bit_cast(pl_v8h, pb), one, 0, 0, 0);
-                }
+                            const uint32_t keep = (in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u);
 #pragma unroll
-                for (int e = 0; e < 16; e++)
-                    acc[db][e] = li == tt ? one[e] : acc[db][e];
+                            for (int db = 0; db < DB; db++)
+                                v[db][st][u][c] &= keep;
+                        }
+            }
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+                const uint4 pb = make_uint4(ph[4 * st], ph[4 * st + 1], ph[4 * st + 2], ph[4 * st + 3]);
+#pragma unroll
+                for (int db = 0; db < DB; db++) {
+                    const uint4 va = make_uint4(v[db][st][0].x, v[db][st][0].y, v[db][st][1].x, v[db][st][1].y);
+                    acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pl_v8h, va),
+                                                                     __builtin_bit_cast(pl_v8h, pb), acc[db], 0, 0, 0);
+                }
+            }
+        });
+
+        // the tiles that waited, a token at a time with the values past it zeroed
+#pragma unroll 1
+        for (int p0 = late; p0 < nmax; p0 += (p0 & 32) ? kPlGroups * kBlock - 32 : 32) {
+            uint32_t ph[8];
+            {
+                pl_v8h k[KS];
+                float s[16];
+                kload(p0, k);
+                score(k, s);
+                probs(p0, s, ph);
+            }
+#pragma unroll 1
+            for (int tt = 0; tt < kPlTok; tt++) {
+                const int own = left(p0, __builtin_amdgcn_readlane(n, tt));
+#pragma unroll
+                for (int db = 0; db < DB; db++) {
+                    pl_v16f one = acc[db];
+#pragma unroll
+                    for (int st = 0; st < 2; st++) {
+                        uint32_t vm[4];
+#pragma unroll
+                        for (int u = 0; u < 2; u++) {
+                            const pl_v2u x = vload(p0, db, st, u);
+#pragma unroll
+                            for (int c = 0; c < 2; c++) {
+                                const int e = 8 * st + 4 * u + 2 * c;
+                                vm[2 * u + c] =
+                                    x[c] & ((in(own, e) ? 0x0000FFFFu : 0u) | (in(own, e + 1) ? 0xFFFF0000u : 0u));
+                            }
+                        }
+                        const uint4 pb = make_uint4(ph[4 * st], ph[4 * st + 1], ph[4 * st + 2], ph[4 * st + 3]);
+                        const uint4 va = make_uint4(vm[0], vm[1], vm[2], vm[3]);
+                        one = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pl_v8h, va),
+                                                                     __builtin_bit_cast(pl_v8h, pb), one, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        acc[db][e] = li == tt ? one[e] : acc[db][e];
+                }
             }
         }
+        if (NW < kPlGroups && group >= NW) {
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    upper[(db * 16 + e) * 64] = acc[db][e];
+                    acc[db][e] = 0.0f;
+                }
+        }
+    }
+    if (NW < kPlGroups) {
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                acc[db][e] = acc[db][e] + upper[(db * 16 + e) * 64];
+        __syncthreads();  // the upper groups' sums are spent
     }
 
     // the wavefronts' sums: the upper half's added to the lower half's
-    __syncthreads();  // the block sums are spent
 #pragma unroll
     for (int half = NW / 2; half > 0; half >>= 1) {
         float *part = sl + (size_t)(wave & (half - 1)) * DB * 16 * 64 + lane;
@@ -848,9 +878,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_prompt_long_kernel(
     }
 }
 
-size_t prompt_long_lds(int hd, int nw, int limit) {
+size_t prompt_long_lds(int hd, int limit) {
     const size_t sums = (size_t)((limit + kBlock - 1) / kBlock) * kPlTok;
-    const size_t parts = (size_t)(nw / 2) * (hd / 32) * 16 * 64, tile = (size_t)kPlTok * (hd + 4);
+    const size_t parts = (size_t)(kPlGroups / 2) * (hd / 32) * 16 * 64, tile = (size_t)kPlTok * (hd + 4);
     return sizeof(float) * std::max(sums, std::max(parts, tile));
 }
 
@@ -858,7 +888,7 @@ size_t prompt_long_lds(int hd, int nw, int limit) {
 
 // The block sums have to fit the LDS, a key-value head's cache a 32-bit offset.
 bool attn_prompt_long_fits(int hd, int limit, int context) {
-    return prompt_long_lds(hd, 8, limit) <= 150 * 1024 && (uint64_t)hd * context * sizeof(uint16_t) <= 1u << 31;
+    return prompt_long_lds(hd, limit) <= 150 * 1024 && (uint64_t)hd * context * sizeof(uint16_t) <= 1u << 31;
 }
 
 // Wavefronts a workgroup: eight while the tiles would leave CUs without one,
@@ -868,8 +898,7 @@ int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, i
                             float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f) {
     const dim3 grid((unsigned)heads, (unsigned)((M + kPlTok - 1) / kPlTok));
     const bool wide = (size_t)grid.x * grid.y <= 2 * (size_t)ctx->cu_count;
-    const int nw = wide ? 8 : 4;
-    const size_t lds = prompt_long_lds(hd, nw, limit);
+    const size_t lds = prompt_long_lds(hd, limit);
 #define GX_PL(HH, WW)                                                                                                \
     attn_prompt_long_kernel<HH, WW><<<grid, 64 * WW, lds, ctx->stream>>>(qh, M, heads, kv_heads, positions, limit,   \
                                                                          kcache, vcache, context, scale, q, scales,  \

@@ -189,12 +189,35 @@ def test_long_prompt_on_exact_scores(dev, orc, hd, heads, kv, M, start, context)
     np.testing.assert_array_equal(qs, q8.reshape(M, -1, 32).astype(np.int32).sum(2))
 
 
-@pytest.mark.parametrize("hd,start", [(128, 1100), (64, 600), (128, 0), (64, 300), (96, 505), (32, 700)])
-def test_long_prompt_keeps_later_infinities_out(dev, hd, start):
+@pytest.mark.parametrize("hd", [32, 128])
+def test_long_prompt_does_not_depend_on_its_batch(dev, hd):
+    """Past 1,024 positions a prompt's token gets the same bits whether its
+    batch is the whole document (four wavefronts a workgroup) or its last
+    tokens (eight, and other tiles)."""
+    heads, kv, n, few = 16, 2, 1060, 41
+    context = (n + 7) // 8 * 8
+    g = synth.rng(hd + 7)
+    k, v, kt, vt = _caches(g, 1, n, kv, hd, context, False)
+    qf = g.standard_normal((n, heads * hd)).astype(np.float16)
+    pos = np.arange(n, dtype=np.int32)
+    args = (kt, vt, heads, kv, hd, n - 1, context)
+    whole = _run(dev, "gx_qwen_attention_parallel", qf, pos, *args)
+    last = _run(dev, "gx_qwen_attention_parallel", np.ascontiguousarray(qf[-few:]), pos[-few:].copy(), *args)
+    for a, b in zip(whole, last):
+        np.testing.assert_array_equal(a[-few:].view(np.uint8), b.view(np.uint8))
+
+
+# LDS and sweeps of eight and (33 tiles of 16 heads) four wavefronts
+WILD = [(128, 1100, 70), (64, 600, 70), (128, 0, 70), (64, 300, 70), (96, 505, 70), (32, 700, 70), (32, 0, 1040),
+        (128, 40, 1060)]
+
+
+@pytest.mark.parametrize("hd,start,M", WILD)
+def test_long_prompt_keeps_later_infinities_out(dev, hd, start, M):
     """An infinite and a NaN value of two tokens in mid-tile: the tokens before
     them get the bits they get without them, the tokens after them everywhere
     but in the blocks of the two elements."""
-    heads, kv, M = 16, 2, 70
+    heads, kv = 16, 2
     n = start + M
     context = (n + 7) // 8 * 8
     g = synth.rng(hd)
