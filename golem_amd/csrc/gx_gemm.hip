@@ -24,6 +24,7 @@
 // product of more than a few tokens, dense or grouped by expert) and an fp16
 // one for callers that hold the activation's fp16 copy.  The weights'
 // nibbles are widened to signed int8 (n - 8) in registers as they are read.
+#include <algorithm>
 #include <type_traits>
 
 #include "gx_device.hpp"
@@ -1023,21 +1024,41 @@ int launch_shape(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8
     return check_launch("q4_0_gemm");
 }
 
-// The shape of a dense product: 128 x 64 where three of its workgroups fall to
-// every CU (a CU holds three), one round whole or more; fewer leave CUs
-// part empty for the length of a whole tile, and 64 x 64 with twice as many
-// wavefronts ends sooner.  9728 x 2560 (us, 128 x 64 / 64 x 64): M = 2048 126
-// / 137, 1000 65 / 72, 500 38.7 / 38.0, 300 27.6 / 24.2; 2560 x 4096 at 1500
-// (480 workgroups) 55.8 / 46.6; 6144 x 2560 at 1500 (1152) 64.1 / 66.9.  Up
-// to 32 tokens half of a 64-token tile would be empty: 128 x 32 (19456 x 2560
-// with SwiGLU at 32: 15.0 against 17.9), as the Q|K|V epilogue has for its
-// small form, whose heads need 128 rows.
+// The shape of a dense product.  Its time goes by the most workgroups any CU
+// takes (in turn or three at once: the matrix core's time a workgroup is the
+// same), so by whole rounds of the CUs: a few tokens or rows more that start a
+// round cost all of it, and which shape needs the fewer, smaller rounds changes
+// from size to size.  A shape's time is taken as a + b rounds, in tenths of a
+// us at 2560 inputs, fitted to 18 matrices of 512 to 32000 rows and 512 to
+// 9728 inputs at 35 token counts from 24 to 2,048: no size takes 3 % more than
+// under the rules before (a count of the workgroups alone) and all 0.7 % more
+// than the fastest shape on average (1.7 % before).  128 x 64 in less than
+// three rounds only with the SwiGLU epilogue: the product's own outputs are
+// four to eight times as many bytes, and three whole tiles a CU then end
+// together.  us 128 x 64 / 64 x 64 / 128 x 32: 19456 x 2560 with SwiGLU at 65
+// tokens 31.2 / 26.3 / 20.5, at 129 34.8 / 35.0 / 29.7, at 257 49.2 / 52.3 /
+// 54.0; 10240 x 2560 with SwiGLU at 560 48.7 / 51.7 / 53.3, at 584 62.6 / 57.8 /
+// 54.3; 9728 x 2560 at 584 56.0 / 48.9 / 50.0, at 2048 126 / 137; 2560 x 4096 at
+// 1500 55.8 / 46.6.  Up to 32 tokens half of a 64-token tile would be empty:
+// 128 x 32 (19456 x 2560 with SwiGLU at 32: 15.0 against 17.9).  The Q|K|V
+// epilogue's heads need 128 rows.
+struct ShapeCost {
+    int rows, tokens, a, b;
+    size_t workgroups(int tiles, int M) const {
+        const int per = rows / kTileRows;
+        return (size_t)((tiles + per - 1) / per) * (size_t)((M + tokens - 1) / tokens);
+    }
+    size_t operator()(gx_ctx *ctx, int tiles, int M) const {
+        return a + b * ((workgroups(tiles, M) + ctx->cu_count - 1) / ctx->cu_count);
+    }
+};
+constexpr ShapeCost kCost128x64{128, 64, 90, 120}, kCost64x64{64, 64, 30, 74}, kCost128x32{128, 32, 60, 78};
+
 template <int EPI>
 int launch_dense(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8_t *q, const float *scales, int M,
                  int row_start, int row_end, const float *bias, float *y, int ldy, int32_t *dots, int8_t *mq,
                  float *ms, int32_t *mqs, const QkvRopeArgs &qr) {
     const int tiles = (row_end + kTileRows - 1) / kTileRows - row_start / kTileRows;
-    const size_t big = (size_t)((tiles + 1) / 2) * ((M + 63) / 64);
 #define GX_SHAPE(SH)                                                                                                 \
     do {                                                                                                             \
         if (EPI == 0 && dots)                                                                                        \
@@ -1046,12 +1067,14 @@ int launch_dense(gx_ctx *ctx, const gx_weight *w, const uint8_t *mat, const int8
         return launch_shape<SH, false, EPI>(ctx, w, mat, q, scales, M, row_start, row_end, bias, y, ldy, nullptr,   \
                                             mq, ms, mqs, qr);                                                       \
     } while (0)
-    if (big >= 3 * (size_t)ctx->cu_count)
-        GX_SHAPE(Shape128x64);
+    const size_t wide = kCost128x64(ctx, tiles, M), narrow = kCost128x32(ctx, tiles, M);
+    const bool whole = EPI == 1 || kCost128x64.workgroups(tiles, M) >= 3 * (size_t)ctx->cu_count;
     if constexpr (EPI != 2) {
-        if (M > 32)
+        if (M > 32 && kCost64x64(ctx, tiles, M) < (whole ? std::min(wide, narrow) : narrow))
             GX_SHAPE(Shape64x64);
     }
+    if (whole && wide < narrow)
+        GX_SHAPE(Shape128x64);
     GX_SHAPE(Shape128x32);
 #undef GX_SHAPE
 }

@@ -18,10 +18,11 @@ def dev():
     d.close()
 
 
-# rows, cols, M, first row, spare floats a row of y: 128 x 64 tiles (from 768
-# workgroups: 98304 rows and more at 64 tokens), 64 x 64, 128 x 32 (to 32
-# tokens); rows past a tile, one block, blocks past a stage and a stretch
-CASES = [(98304 + 65, 64, 64, 0, 0), (49152, 32, 65, 31, 3), (65, 32, 33, 0, 0), (1000, 2080, 65, 3, 1),
+# rows, cols, M, first row, spare floats a row of y: 128 x 64 tiles (three
+# whole rounds of 256 CUs, the last row tile and the last token part full), 64 x
+# 64, 128 x 32 (to 32 tokens, and where the others need another round); rows
+# past a tile, one block, blocks past a stage and a stretch
+CASES = [(98304 - 63, 64, 63, 0, 0), (6000, 64, 129, 5, 1), (98304 + 65, 64, 64, 0, 0), (49152, 32, 65, 31, 3), (65, 32, 33, 0, 0), (1000, 2080, 65, 3, 1),
          (192, 4128, 130, 0, 4), (64, 288, 64, 0, 0), (1000, 96, 32, 64, 2), (129, 2592, 17, 0, 0)]
 
 
