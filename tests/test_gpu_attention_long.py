@@ -66,9 +66,10 @@ def _oracle(orc, fn, qf, k, v, pos, slots, rows, heads, kv, hd):
     return want
 
 
-# head width, heads, key-value heads, positions (block, run and piece edges)
+# head width, heads, key-value heads, positions (block, run and piece edges;
+# past 16,384 positions a second 256 blocks' sums, several pieces a workgroup)
 DECODE = [(128, 8, 2, [768]), (128, 4, 4, [1500, 63, 64]), (64, 4, 2, [2100, 0]), (32, 8, 1, [1023, 1024, 31, 32]),
-          (96, 4, 2, [801])]
+          (96, 4, 2, [801]), (32, 2, 1, [16383, 16384, 16500]), (32, 32, 8, [33000, 70, 16400, 20000])]
 
 
 @pytest.mark.parametrize("hd,heads,kv,positions", DECODE)
@@ -162,9 +163,11 @@ def test_long_decode_forms(dev, orc, hd, heads, kv, M, n):
 
 
 # head width, heads, key-value heads, M, first position, context: few tiles
-# (eight wavefronts) and many (four), ragged tiles, one token past 1024
+# (eight wavefronts) and many (four), ragged tiles, one token past 1024; block
+# sums past 64 KB of LDS, and the most that fit it
 PROMPT = [(128, 4, 1, 33, 1100, 1144), (64, 4, 2, 70, 990, 1064), (32, 8, 1, 5, 1020, 1032), (96, 4, 4, 64, 1500, 1568),
-          (32, 32, 8, 544, 600, 1160), (128, 32, 8, 530, 500, 1032)]
+          (32, 32, 8, 544, 600, 1160), (128, 32, 8, 530, 500, 1032), (32, 2, 1, 5, 33000, 33008),
+          (64, 2, 2, 6, 76794, 76800)]
 
 
 @pytest.mark.parametrize("hd,heads,kv,M,start,context", PROMPT)
@@ -187,6 +190,19 @@ def test_long_prompt_on_exact_scores(dev, orc, hd, heads, kv, M, start, context)
     assert np.abs(dq).max() <= 1 and np.count_nonzero(dq) <= max(3, dq.size // 1000)
     assert np.abs(sc[rows] / want.scales_rows() - 1).max() <= 2.0 ** -10
     np.testing.assert_array_equal(qs, q8.reshape(M, -1, 32).astype(np.int32).sum(2))
+
+
+def test_prompt_past_the_sweeps_runs_the_serial_passes(dev):
+    """A position more than the block sums' LDS holds."""
+    hd, heads, kv, M, n = 32, 2, 1, 5, 76801
+    context = (n + 7) // 8 * 8
+    g = synth.rng(8)
+    k, v, kt, vt = _caches(g, 1, n, kv, hd, context, False)
+    qf = g.standard_normal((M, heads * hd)).astype(np.float16)
+    pos = np.arange(n - M, n, dtype=np.int32)
+    args = (qf, pos, kt, vt, heads, kv, hd, n - 1, context)
+    for a, b in zip(_run(dev, "gx_qwen_attention_parallel", *args), _run(dev, "gx_qwen_attention", *args)):
+        np.testing.assert_array_equal(a.view(np.uint8), b.view(np.uint8))
 
 
 @pytest.mark.parametrize("hd", [32, 128])
