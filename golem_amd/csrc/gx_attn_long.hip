@@ -1,9 +1,9 @@
 // gx_attn_long.hip - the parallel-order attention past the prefixes that one
 // workgroup holds (gx_qwen.hip): a decode step's positions spread over the
-// chip, and a prompt's attention on the matrix cores with nothing but the
-// block sums kept between its sweeps.
+// chip, or a workgroup a token and a few of its heads; and a prompt's attention
+// on the matrix cores with nothing but the block sums kept between its sweeps.
 //
-// Both compute what the short forms compute (qwen/attention.go:96-124,
+// All compute what the short forms compute (qwen/attention.go:96-124,
 // nn/ops.go:59-73): the scores, their maximum, the float64 exponential of the
 // float difference rounded to float (exp_neg), the total as 64-position blocks
 // summed pairwise and the blocks added in order, the probabilities divided
@@ -480,7 +480,8 @@ __global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
 //
 // grid (heads, ceil(M / 32)), a workgroup per (query head, 32-token tile), NW
 // wavefronts, each with its own 64-position blocks of the prefix (block b:
-// wavefront b % NW).  The scores are taken transposed, positions by tokens
+// wavefront b % NW; of the last sweep's values, the groups b % 8 that leave the
+// wavefront's number when divided by NW).  The scores are taken transposed, positions by tokens
 // (v_mfma_f32_32x32x16_f16, the keys as the row operand): a lane then holds
 // sixteen positions of one token, so that
 //   - the token's maximum and the pairwise block sums are sums over the lane's
@@ -499,8 +500,9 @@ __global__ __launch_bounds__(kRowsThreads) void attn_rows_kernel(
 // from the L2.  The value sums of the eight groups of blocks (b % 8) are added
 // pairwise at the end (c + 4, then c + 2, c + 1).
 // What bounds it: the exponentials (float64, twice) and the MFMAs, about 900
-// and 300 cycles a 32 x 32 tile and sweep.  1,500 tokens of 32 heads: 172 us,
-// where the serial passes took 679 (scores 226, softmax 132, values 321).
+// and 300 cycles a 32 x 32 tile and sweep.  1,500 tokens of 32 heads: 154 us in
+// a replayed graph, where the serial passes took 679 (scores 226, softmax 132,
+// values 321).
 typedef _Float16 pl_v8h __attribute__((ext_vector_type(8)));
 typedef float pl_v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t pl_v2u __attribute__((ext_vector_type(2)));
@@ -891,8 +893,10 @@ bool attn_prompt_long_fits(int hd, int limit, int context) {
     return prompt_long_lds(hd, limit) <= 150 * 1024 && (uint64_t)hd * context * sizeof(uint16_t) <= 1u << 31;
 }
 
-// Wavefronts a workgroup: eight while the tiles would leave CUs without one,
-// four (two workgroups a CU) otherwise.
+// Wavefronts a workgroup: eight to two workgroups a CU, four past that (us 8 /
+// 4 at 1,100 positions: 32 heads of 128 256 tokens 48 / 57, 500 74 / 69, 544 95
+// / 85, 1,000 113 / 102; 16 heads of 128 768 tokens 59 / 62; 32 of 64 512
+// tokens 50 / 55, 1,000 69 / 70; the same bits).
 int launch_attn_prompt_long(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int hd, int limit,
                             const int32_t *positions, const uint16_t *kcache, const uint16_t *vcache, int context,
                             float scale, int8_t *q, float *scales, int32_t *qsum, float *heads_f) {

@@ -172,7 +172,7 @@ int gx_matmul_q4_0_expert(gx_ctx *ctx, const gx_weight *w, int expert, const int
 /* y[m][r] = W[r] . x[m] (+ bias[r]) for a Q6_K matrix and a Q8_K batch:
  * MatVecQ6_K and matVecQ6_KRows (nn/dot_q6_k.go:64-103), which include the
  * two-column dotQ6_Kx2 (nn/dot_q6_k_amd64.go:14-20): one weight read serves
- * sixteen columns.  Bit-identical to golem's dotQ6_KGo. */
+ * up to sixteen columns.  Bit-identical to golem's dotQ6_KGo. */
 int gx_matmul_q6_k(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const float *kscales, const int16_t *bsums,
                    int M, int row_start, int row_end, const float *bias, float *y, int ldy);
 
@@ -392,8 +392,13 @@ int gx_qwen_qkv_rope(gx_ctx *ctx, const gx_weight *w, const int8_t *q, const flo
                      uint16_t *kcache, uint16_t *vcache, int context, const int32_t *slots, int nslots,
                      float *qkv);
 
-/* Device bytes of the workspace gx_qwen_attention needs for M positions of
- * `heads` query heads whose positions are at most max_pos. */
+/* Device bytes of the workspace gx_qwen_attention and
+ * gx_qwen_attention_parallel take for M positions of `heads` query heads whose
+ * positions are at most max_pos.  From max_pos 768 on it holds, past the
+ * M * heads rows of scores and probabilities that the serial passes need, the
+ * partial value sums of a decode step's positions spread over the chip (16
+ * bytes a row and position for up to 16 of the M tokens).  gx_qwen_attention,
+ * and prompts, run with the rows alone. */
 int gx_qwen_attention_workspace_bytes(int M, int heads, int max_pos, size_t *bytes);
 
 /* The attention proper (qwen/attention.go:86-124) for M positions: every
@@ -446,18 +451,29 @@ int gx_qwen_rope_attention(gx_ctx *ctx, const float *qkv, int ldqkv, int heads, 
  * thread of a workgroup takes a share of both sums, where golem's order
  * leaves them to one lane per head and one per head element.  Same
  * arguments, caches and outputs as the serial forms; the caches come out bit
- * for bit the same.  A decode step past 768 positions runs as four launches
- * spread over the prefix, the same order and so the same bits; it needs the
- * whole of gx_qwen_attention_workspace_bytes (with what the serial passes
- * need alone, M * heads rows of scores and probabilities, they run instead).
+ * for bit the same.
+ *
+ * A decode step past 768 positions takes the same order and so gives the same
+ * bits, alone or with other conversations, however far max_pos lies above its
+ * position; it runs as one launch or, few tokens far in, as four spread over
+ * the prefix.  It needs the whole of gx_qwen_attention_workspace_bytes: with
+ * the serial passes' rows alone it runs as them, or, one conversation's tokens
+ * to 1024 positions, as a prompt.  A negative position sees the first position
+ * while max_pos is below 768 (1024 for one conversation's tokens), and past
+ * that none: zeros.
+ *
  * A prompt (M > 4 tokens of one conversation) runs on the matrix cores: the
  * scores and the value sums are fp16 MFMA products (exact products, fp32 sums
  * in the matrix core's order), the maximum, exponentials, total and fp16
  * probabilities as above; the head outputs stay within 1e-4 of RMS of
- * golem's.  Past 1024 positions (past 576 where more than 32 workgroups
- * share the work) it sweeps the prefix three times instead of keeping the
- * scores, to about 76,000 positions; longer prompts take the serial
- * kernels. */
+ * golem's, and an infinite or NaN value reaches only the tokens that see it.
+ * To 1024 positions it keeps the scores in LDS or, where that is the faster
+ * (past 576 positions, by the heads, their width and how early the tokens
+ * are), sweeps the prefix three times; past 1024 it sweeps, to 76,800
+ * positions; longer prompts take the serial kernels.  The two group the value
+ * sums differently, and the LDS form by its 32-token tiles' prefixes, so to
+ * 1024 positions a token's last bits can depend on its batch; past them they
+ * do not. */
 int gx_qwen_attention_parallel(gx_ctx *ctx, const uint16_t *qh, int M, int heads, int kv_heads, int head_dim,
                                int max_pos, const int32_t *positions, const uint16_t *kcache,
                                const uint16_t *vcache, int context, int8_t *q, float *scales, int32_t *qsum,
