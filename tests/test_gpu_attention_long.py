@@ -1,7 +1,7 @@
 """The parallel-order attention past one workgroup's prefixes: a decode step
-spread over the chip (prefixes beyond 768, tokens of several conversations)
-and a prompt on the matrix cores in three sweeps (prefixes beyond 1024),
-against the oracle's restatement of the order."""
+spread over the chip or a workgroup a token's heads (prefixes beyond 768, tokens
+of several conversations) and a prompt on the matrix cores in three sweeps
+(prefixes beyond 1024), against the oracle's restatement of the order."""
 import math
 
 import numpy as np
@@ -130,6 +130,21 @@ def test_negative_positions_of_a_lone_conversation(dev, orc, M, n):
     np.testing.assert_array_equal(q8, want.q_rows())
     np.testing.assert_array_equal(_bits(sc), _bits(want.scales_rows()))
     np.testing.assert_array_equal(qs, want.qsum_rows())
+
+
+def test_rows_alone_of_a_lone_conversation(dev):
+    """With the serial passes' workspace alone, two tokens to 1,024 positions
+    run as the end of a prompt."""
+    hd, heads, kv, n, context = 64, 4, 2, 900, 904
+    g = synth.rng(17)
+    k, v, kt, vt = _caches(g, 1, n, kv, hd, context, False)
+    qf = g.standard_normal((6, heads * hd)).astype(np.float16)
+    pos = np.arange(n - 6, n, dtype=np.int32)
+    args = (kt, vt, heads, kv, hd, n - 1, context)
+    prompt = _run(dev, "gx_qwen_attention_parallel", qf, pos, *args)
+    two = _run(dev, "gx_qwen_attention_parallel", np.ascontiguousarray(qf[4:]), pos[4:].copy(), *args, least=True)
+    for a, b in zip(prompt, two):
+        np.testing.assert_array_equal(a[4:].view(np.uint8), b.view(np.uint8))
 
 
 # head width, heads, key-value heads, tokens, longest prefix.  A workgroup a
